@@ -101,3 +101,26 @@ def test_product_graded_from_producer_statistic(M, dtype):
     torch.cuda.synchronize()
     assert torch.equal(torch.isnan(a), torch.isnan(b))
     assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("M,K", [(2064, 4104), (1030, 8192), (17, 520)])
+def test_large_batches(M, K, dtype):
+    """Batches whose blocks take several 512-column pieces (the norm) or four
+    rows per wave (the activation), ragged at the last piece and the last rows."""
+    from grinqh.producer import rmsnorm_sigma, silu_mul_sigma
+    rng = np.random.default_rng(M * K)
+    x, r, w = _rand(rng, (M, K), dtype, 3.0), _rand(rng, (M, K), dtype), _rand(rng, (K,), dtype)
+    y, sig, h = rmsnorm_sigma(x, w, 1e-5, r)
+    a, asig = silu_mul_sigma(torch.cat((x, r), -1))
+    torch.cuda.synchronize()
+    href = (x.float() + r.float()).to(DT[dtype])
+    assert torch.equal(h, href), "residual sum"
+    hf = href.float()
+    yref = (hf * torch.rsqrt(hf.pow(2).mean(-1, keepdim=True) + 1e-5)).to(DT[dtype]).float() * w.float()
+    # as above: one unit of roundoff of the normalised value, one of y, from the variance's summation order
+    assert bool(((y.float() - yref).abs() <= 4 * U[dtype] * yref.abs() + 1e-6).all())
+    np.testing.assert_array_equal(sig.cpu().numpy(), _chunk_max(y))
+    act = (x.float() / (1 + torch.exp(-x.float()))).to(DT[dtype]).float() * r.float()
+    assert bool(((a.float() - act).abs() <= 4 * U[dtype] * act.abs() + 1e-6).all())
+    np.testing.assert_array_equal(asig.cpu().numpy(), _chunk_max(a))
