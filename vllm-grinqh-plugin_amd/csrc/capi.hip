@@ -62,7 +62,6 @@ struct WorkspaceLayout {
   bool tall;       // the large-batch prefill kernel serves the product (prefill_tall.hip)
   TallPlan tall_plan;
   size_t xt_off;   // its repacked activations (after the partial sums)
-  DecodePlan plan;
 };
 
 // Which kernel serves a large batch that both can.  Measured on MI355X
@@ -81,8 +80,8 @@ bool prefill_prefers_library(int64_t M, int64_t K, int64_t N) {
 
 // Plan of one launch of mc rows: the GEMV kernel up to kGemvMaxRows rows, the
 // decode kernel above.  group_size 32 gives the largest GEMV workspace.
-DecodePlan plan_launch(int64_t mc, int64_t K, int64_t N, int64_t group_size) {
-  return mc <= kGemvMaxRows ? plan_gemv(mc, K, N, group_size) : plan_decode(mc, K, N);
+DecodePlan plan_launch(int64_t mc, int64_t K, int64_t N, int64_t group_size, int max_bits, bool dense, bool wide) {
+  return mc <= kGemvMaxRows ? plan_gemv(mc, K, N, group_size) : plan_decode(mc, K, N, max_bits, dense, wide);
 }
 int launch_main(const DecodeParams& p, const DecodePlan& plan, int max_bits, int dtype, bool dense,
                 hipStream_t st) {
@@ -122,8 +121,11 @@ WorkspaceLayout layout_for(int64_t M, int64_t K, int64_t N, int mode, bool allow
                          (tall_fits ? lib_f16 && lib_bf16 && prefill_prefers_library(M, K, N) : lib_f16 || lib_bf16);
   bool tall_shape = false;
   if (M <= kDecodeMaxRows) {
-    w.plan = plan_launch(M > 0 ? M : 1, K, N, 32);
-    partial = w.plan.splits > 1 ? w.plan.workspace : 0;
+    for (const int bits : {2, 8})  // any bit width's plan fits, whatever the planes' alignment
+      for (const bool wide : {false, true}) {
+        const DecodePlan plan = plan_launch(M > 0 ? M : 1, K, N, 32, bits, !g, wide);
+        partial = plan.splits > 1 && plan.workspace > partial ? plan.workspace : partial;
+      }
   } else {  // prefill: partial sums only when its grid is split over K
     tall_shape = !lib_first && tall_fits;
     xt = tall_shape ? round_up(tall_x_bytes(M, K), 256) : 0;
@@ -378,13 +380,14 @@ int run_product(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int
   }  // else the GEMV and decode kernels reduce the batch statistic of their rows themselves
   for (int64_t m0 = 0; m0 < M; m0 += rows_per_launch) {
     const int64_t mc = (M - m0) < rows_per_launch ? (M - m0) : rows_per_launch;
-    const DecodePlan plan = plan_launch(mc, K, N, group_size);
+    const bool wide = N % 64 == 0 && aligned(planes, 16);
+    const DecodePlan plan = plan_launch(mc, K, N, group_size, max_bits, !graded, wide);
     p.x = xs + m0 * ldx;
     p.y = ys + m0 * N;
     p.M = (int)mc;
     p.splits = plan.splits;
     p.tiles_per_split = plan.tiles_per_split;
-    const int64_t block_cols = mc <= kGemvMaxRows ? 1024 : 256;  // logical columns per column block
+    const int64_t block_cols = mc <= kGemvMaxRows ? 1024 : 256 * plan.cg;  // logical columns per column block
     p.counters =
         splitk_in_kernel(plan, mc, N, block_cols) ? reinterpret_cast<uint32_t*>(ws + wl.counter_off) : nullptr;
     if (m0 == 0) arm_kernel_timing();

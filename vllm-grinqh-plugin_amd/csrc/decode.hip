@@ -8,26 +8,36 @@
 //
 // Work decomposition
 //   block   = (column block, K range), one-dimensional grid renumbered per XCD
-//   column block: 16 plane-word columns w0..w0+15 = 256 logical columns (16
-//             column tiles r of 16 contiguous columns r*NW + w0 + c); two
-//             neighbours share every 128-byte line of the planes
+//   column block: 16 or 32 plane-word columns (CG groups of 16): 256 or 512
+//             logical columns (16 column tiles r, columns r*NW + w0 + c)
 //   K range = `tiles_per_split` 32-row tiles (split-K)
-//   waves   = groups of output dwords j x K sub-ranges: 8 waves (two per
-//             SIMD) as 2 dword pairs x 4 sub-ranges for 5-16 rows and for
-//             17-64 rows in fp16; 4 waves as MT dword groups x 4/MT
-//             sub-ranges for 17-64 rows in bf16
+//   waves   = 8 (two per SIMD): CG column groups x JG groups of output dwords
+//             j x KW K sub-ranges; the CG * JG waves of a sub-range share its
+//             tiles
 //
-// Phase 1 (whole block): stage the scales (and, up to 16 rows, x[:, K range])
-// in LDS, grade every row (sigma = max_m |x|, zone bits, midpoint bias) and
-// precompute each (row, plane) byte offset, with bit 31 set for planes the
-// row does not need.
+// What bounds it: at small shapes the launch, the prologue and the split-K
+// completion (about 10 us in all); in the loop, dense, the plane traffic, and
+// graded the unpacking VALU.  The plane words come through LDS by direct
+// buffer-to-LDS loads because of the traffic: with every wave loading its own
+// tiles into registers, the two waves that share a tile requested it twice, and
+// a stream of the same requests without arithmetic reached 2.1 TB/s (gate_up,
+// one MI355X); each tile requested once through 16-byte LDS loads reaches 3.4
+// TB/s with 16 word columns per block, 4.6 with 32, 5.4 with 64 (longer runs
+// of each plane line per block; a plain copy: 5.1).  The registers this frees
+// took bf16 above 16 rows from four waves per block to eight.  Measured,
+// product with its reduction: gate_up 16 rows dense 59.6 -> 36.2 us, 64 rows
+// 66.9 -> 58.8, in bf16 104.5 -> 56; Llama-3-70B gate_up 16 rows 178 -> 128.
 //
-// Phase 2 (per wave): for each tile, each lane (c = lane&15, q = lane>>4) loads
-// one 32-bit plane word per (row, plane) of its 8 rows with raw buffer loads;
-// offsets with bit 31 set fall past the buffer end and return 0 without a
-// memory access, so only the planes a row needs are fetched and no load is
-// branched around.  One or two tiles of loads stay in flight while the
-// current tile is unpacked.  Code bytes are rebuilt branch-free:
+// Phase 1 (whole block): reduce the batch statistic of the block's rows from x
+// (unless given), grade every row (sigma = max_m |x|: zone bits, midpoint
+// bias), load the scales into LDS.
+//
+// Phase 2 (per wave): each wave of a K sub-range loads a share of the tiles'
+// plane words and x straight into LDS, one or two tiles ahead; a (row, plane)
+// the grading does not need has an offset past the buffer end, which leaves
+// zeros without a memory access.  A handshake through LDS flags per tile says
+// that all shares have arrived; then lane (c = lane & 15, q = lane >> 4) reads
+// the 8 x Z words of its 8 rows.  Code bytes are rebuilt branch-free:
 // G_z = rot(D_z, 2z), H_j = field merge of the G_z, V_j = rot(H_j, -2j); then
 // turned into the MFMA B operand in one of two ways:
 //   - code bytes (5-16 rows, and bf16): fp16 B = u as the subnormal u*2^-24
@@ -38,12 +48,6 @@
 //     in fp32, as grinqh/kernel.py:148-158 applies scales;
 //   - the scaled weight (17-64 rows in fp16): B = RNE(w_eff * s) in fp16,
 //     accumulated straight into y (no per-group sums, no correction column).
-// Above 16 rows the A operand (x) is not staged for the whole K range: in
-// fp16 the two waves that share a K sub-range each load half of the next
-// tile's x straight into LDS (buffer loads to LDS) and read the whole tile
-// from there, after a per-tile handshake through LDS flags, so each x tile is
-// fetched once per K sub-range instead of once per wave; bf16 loads it from
-// L2 with the tile's plane words.
 //
 // Split-K partials are reduced deterministically: the K sub-ranges of a block
 // through LDS in fixed order; the K ranges of the grid either by the range
@@ -56,101 +60,88 @@
 
 namespace grinqh {
 
-constexpr int kDecodeRowsPerBlock = 2048;  // rows per block at MT = 1 (x staged in LDS)
-
 // 17-64 rows in fp16 ("scaled" path) multiply the scaled weight RNE(w * s),
 // built in registers as the prefill builds it in LDS, and accumulate the
 // output directly: no per-group partial sums, no correction column, no group
 // epilogue.  The registers this frees let a wave cover two output dwords of all
-// 64 rows (128 sums per lane), so the eight waves are two output-dword pairs x
-// four K sub-ranges: each plane word and x element is loaded and unpacked by
-// two waves (one per dword pair) instead of four.  The weight is rounded once to fp16, as in the
-// reference's dense path (grinqh/kernel.py:586).
+// 64 rows (128 sums per lane); in bf16 a wave covers two dwords of 32 rows or
+// one of 64.  The weight is rounded once to fp16, as in the reference's dense
+// path (grinqh/kernel.py:586).
 template <typename DT, int MT>
 constexpr bool decode_scaled() { return MT >= 2 && DT::id == F16::id; }
+
+constexpr int kDecodeWaves = 8;
+// K rows a block can hold (scales, grades)
+constexpr int decode_rows_per_block(int cg) { return cg == 2 ? 1024 : 2048; }
+// groups of output dwords among a block's waves (4 / this dwords per wave)
 template <typename DT, int MT>
-constexpr int decode_waves() { return (decode_scaled<DT, MT>() || MT == 1) ? 8 : 4; }
+constexpr int decode_dword_groups() { return !decode_scaled<DT, MT>() && MT == 4 ? 4 : 2; }
 
-template <typename DT, int MT, int Z, bool DENSE>
-__global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kernel(DecodeParams p) {
+// CG: groups of 16 word columns per block.  WIDE: plane rows 16-byte aligned
+// (16-byte loads of four words), else 4-byte loads
+template <typename DT, int MT, int Z, bool DENSE, bool WIDE, int CG>
+__global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodeParams p) {
   constexpr bool SC = decode_scaled<DT, MT>();
-  constexpr int NWV = decode_waves<DT, MT>();
+  constexpr int NWV = kDecodeWaves;
   constexpr int NT = 64 * NWV;         // threads per block
-  constexpr int MP = 16 * MT;          // padded rows of x
-  constexpr int NJ = NWV == 8 ? 2 : 4 / MT;  // output dwords j per wave
-  constexpr int KW = NWV == 8 ? 4 : 4 / MT;  // K sub-ranges per block
-  constexpr int JG = NWV / KW;         // groups of output dwords (waves per K sub-range)
-  // tiles of loads in flight ahead of the one unpacked; the scaled path runs
-  // two waves per SIMD on 256 registers, with one tile ahead (33-64 rows) or
-  // two (17-32 rows), and its A operand through LDS
-  constexpr int PF = (SC && MT == 4) ? 1 : 2;
-  // 17-64 rows in fp16: the JG waves of a K sub-range share its x tiles
-  // through LDS (see s_xr0), each loading XF of a tile's MT fragments.  bf16
-  // (one wave per SIMD, none to cover a wave's wait at the handshake) loads
-  // them with the plane words two tiles ahead: shared, its 48-64-row
-  // products took 17-25 % longer.
-  constexpr bool XL = SC;
-  constexpr int XF = MT / JG;
-  static_assert(!XL || (XF >= 1 && XF * JG == MT), "each wave of a K sub-range loads whole fragments");
+  constexpr int WB = 16 * CG;          // plane-word columns per block
+  constexpr int JG = decode_dword_groups<DT, MT>();
+  constexpr int NJ = 4 / JG;           // output dwords j per wave
+  constexpr int SG = CG * JG;          // waves per K sub-range
+  constexpr int KW = NWV / SG;         // K sub-ranges per block
   constexpr int SH = 8 - 2 * Z;
-  // Up to 16 rows x is staged in LDS for the block's K range; above that the
-  // A operand comes tile by tile from global memory (L2-resident; through the
-  // shared LDS slots in fp16, with the plane words in bf16), and grading
-  // uses the batch statistic of the block's rows, reduced from x
-  // in the prologue (or given by the caller), so the K range is not limited
-  // by staging x.
-  constexpr bool AG = MT >= 2;
-  constexpr int RMAX = AG ? kDecodeRowsPerBlock : kDecodeRowsPerBlock / MT;
-  static_assert(!AG || RMAX / 8 <= 64 * decode_waves<DT, MT>(), "one statistic chunk per thread");
-  constexpr int XS = RMAX + 8;  // halves per staged x row (16-byte rows, banks staggered)
-  constexpr int X_BYTES = AG ? 0 : MP * XS * 2;
-  constexpr int OFF_BYTES = RMAX * Z * 4;
-  // f32x4 slots for the in-block reduction, done one m-tile at a time
-  constexpr int RED_VECS = (KW - 1) * JG * NJ * 4 * 64;
-  constexpr int POOL_BYTES = (X_BYTES + OFF_BYTES) > RED_VECS * 16 ? (X_BYTES + OFF_BYTES) : RED_VECS * 16;
+  constexpr int RMAX = decode_rows_per_block(CG);
+  static_assert(RMAX / 8 <= NT, "one statistic chunk per thread");
   constexpr int SC_GROUPS = RMAX / 32 + 1;  // scale groups a K range can touch (group size >= 32)
-  constexpr int CPR = RMAX / 8;             // 16-byte x chunks per staged row
-  constexpr int XPT = AG ? 1 : MP * CPR / NT;  // x chunks per thread
-  constexpr int SPT = (SC_GROUPS * 32 + NT - 1) / NT;  // 16-byte scale chunks per thread
+  constexpr int SPT = CG == 2 ? 3 : 2;      // 16-byte scale chunks a thread keeps in flight
 
-  // staging area: x rows and (row, plane) offsets; reused for the in-block reduction
-  __shared__ __align__(16) unsigned char s_pool[POOL_BYTES];
-  __shared__ __align__(16) uint16_t s_bv[RMAX];    // row -> correction-column value
-  __shared__ __align__(16) uint32_t s_xm[RMAX];    // row -> zone-0 flip
-  __shared__ __align__(16) uint16_t s_scale[SC_GROUPS * 256];  // (group, tile, column) scales
+  // Plane words and x of each K sub-range's tiles come into LDS by direct
+  // buffer-to-LDS loads, PF tiles ahead, each wave of the sub-range loading a
+  // share, in PF + 1 slots (one per tile of the unrolled loop) that are
+  // separate LDS arrays, so that the compiler's wait for one slot's loads does
+  // not also wait for the others'.  A plane slot holds, per sub-range,
+  // [row in octet e][zone z][octet q][word column]: lane (c, q) reads its 8 x Z
+  // words at one offset plus constants, without bank conflicts (with 32 word
+  // columns the two halves are swapped for odd q).
+  constexpr int PF = (MT == 4 && SC ? 1 : 2);
+  constexpr int GB = WIDE ? 4 : 1;                   // words per lane and load
+  constexpr int TILE = 32 * Z * WB * 4;              // bytes of one sub-range's tile
+  constexpr int IPT = TILE / (64 * GB * 4);          // loads per tile
+  constexpr int IPW = (IPT + SG - 1) / SG;           // at most per wave
+  constexpr int XPW = (MT + SG - 1) / SG;            // x fragments per wave, at most
+  constexpr int RED_SLOT = NJ * 4 * 64 * 16;         // one wave's sums of an m-tile
+  constexpr int RED_SLOTS = (KW - 1) * SG;
+  constexpr int RED_ARRAYS = PF + 1;
+  constexpr int RED_PER = (RED_SLOTS + RED_ARRAYS - 1) / RED_ARRAYS;
+  constexpr int PL_BYTES = KW * TILE > RED_PER * RED_SLOT ? KW * TILE : RED_PER * RED_SLOT;
+  constexpr int XR_BYTES = KW * MT * 1024;
+  constexpr int SIG_BYTES = NT * 8 * 4;  // at most NT / U slices of U chunks of 8 rows
+  __shared__ __align__(16) unsigned char s_pl0[PL_BYTES > SIG_BYTES ? PL_BYTES : SIG_BYTES];
+  __shared__ __align__(16) unsigned char s_pl1[PL_BYTES];
+  __shared__ __align__(16) unsigned char s_pl2[PF == 2 ? PL_BYTES : 16];
+  __shared__ __align__(16) unsigned char s_xr0[XR_BYTES];
+  __shared__ __align__(16) unsigned char s_xr1[XR_BYTES];
+  __shared__ __align__(16) unsigned char s_xr2[PF == 2 ? XR_BYTES : 16];
+  __shared__ __align__(16) uint16_t s_bv[DENSE ? 8 : RMAX];  // row -> correction-column value, or -c_row
+  __shared__ __align__(16) uint8_t s_zb[DENSE ? 16 : RMAX];  // row -> zone bits
+  __shared__ __align__(16) uint16_t s_scale[SC_GROUPS * 16 * WB];  // (group, tile, column) scales
   __shared__ uint32_t s_smax;  // graded scaled path: largest |scale| (fp16 bits) above the overflow limit
-  // above 16 rows, graded, no statistic given: this block's rows of the batch
-  // statistic, max_m |x[m][k]| as float bits (an entry that is NaN in every
-  // row gives 0; every output of such a batch is NaN whatever its grading)
-  // 17-64 rows in fp16: the x tile of each K sub-range (the A operand of its
-  // JG waves) comes into LDS by direct buffer-to-LDS loads one tile ahead,
-  // each wave loading XF of its fragments, in PF + 1 slots (one per tile buffer of
-  // the unrolled loop) that are separate LDS arrays (so that the compiler's
-  // wait for one slot's loads does not also wait for the others').
-  // s_xflag[w] is the last tile whose half wave w has in LDS.  The statistic
-  // above shares the first slot's storage: it is read only before the first
-  // of those loads.
-  constexpr int XR_BYTES = XL ? KW * MT * 1024 : 0;
-  constexpr int SIG_BYTES = AG ? RMAX * 4 : 4;
-  __shared__ __align__(16) unsigned char s_xr0[XR_BYTES > SIG_BYTES ? XR_BYTES : SIG_BYTES];
-  __shared__ __align__(16) unsigned char s_xr1[XR_BYTES > 16 ? XR_BYTES : 16];
-  __shared__ __align__(16) unsigned char s_xr2[(XL && PF == 2 && XR_BYTES > 16) ? XR_BYTES : 16];
-  __shared__ int s_xflag[NWV];
-  uint32_t* s_sig = reinterpret_cast<uint32_t*>(s_xr0);
-  uint16_t* s_x = reinterpret_cast<uint16_t*>(s_pool);
-  uint32_t* s_off = reinterpret_cast<uint32_t*>(s_pool + X_BYTES);
-  f32x4_t* s_red = reinterpret_cast<f32x4_t*>(s_pool);
+  __shared__ int s_flag[NWV];  // the last tile whose share wave w has in LDS
+  // graded, no statistic given: max |x[m][k]| per slice of the batch rows (an
+  // entry that is NaN in every row gives 0; every output of such a batch is NaN)
+  float* s_sig = reinterpret_cast<float*>(s_pl0);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform
-  const int jg = wave % JG, kw = wave / JG;
-  if (XL && lane == 0) s_xflag[wave] = -(1 << 30);  // read by the partner only after the next barrier
+  const int jg = wave % JG, cg = (wave / JG) % CG, kw = wave / SG;
+  const int sw = wave % SG;  // this wave among those of its K sub-range
+  if (lane == 0) s_flag[wave] = -(1 << 30);  // read by the others only after the next barrier
   const int c = lane & 15, q = lane >> 4;
   // logical block = (column block, K range), column blocks fastest, ranges of
   // consecutive logical blocks per XCD (adjacent column blocks share lines)
-  const int col_blocks = (p.NW + 15) >> 4;
+  const int col_blocks = (p.NW + WB - 1) / WB;
   const int lb = xcd_chunked(blockIdx.x, gridDim.x);
-  const int w0 = (lb % col_blocks) * 16;
+  const int w0 = (lb % col_blocks) * WB;
   const int split = lb / col_blocks;
   const int ntiles_total = p.K >> 5;
   const int tile0 = split * p.tiles_per_split;
@@ -169,20 +160,15 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
   constexpr uint32_t kScaleLimit = 0x7BFFu - ((uint32_t)(2 * Z - 1) << 10);  // 65504 / 2^(2Z-1), fp16 bits
   uint32_t smax = 0;  // largest |scale| bits this thread staged
   if (GUARD && threadIdx.x == 0) s_smax = 0;
-  const bool own_sigma = AG && !DENSE && p.sigma == nullptr;  // block-uniform
-  if (own_sigma)
-    for (int i = tid; i < R; i += NT) s_sig[i] = 0u;
+  const bool own_sigma = !DENSE && p.sigma == nullptr;  // block-uniform
+  const int sig_slices = min(NT / (R >> 3), p.M);  // batch rows are dealt to this many threads per K chunk
 
-  float sig_part[8];  // this thread's maxima of K chunk sig_chunk (-1: none)
-  int sig_chunk = -1;
-
-  // ---- phase 1a: stage x[:, row0 .. row0+R) in LDS (up to 16 rows) or reduce
-  // the block's statistic from it, and load the scales.  The scales are stored
-  // to LDS only once the first tiles' plane loads are issued, so their memory
-  // round trip overlaps those loads; they are loaded after every x load, so
-  // that waiting for x does not wait for them.  Out-of-range buffer offsets
-  // read 0: rows m >= M stage as zeros, and nothing past the end of x or the
-  // scale array is touched.
+  // ---- phase 1a: reduce the block's statistic from x and load the scales.
+  // The scales are stored to LDS only once the first tiles' loads are issued,
+  // so their memory round trip overlaps those loads; they are loaded after
+  // every x load, so that waiting for x does not wait for them.  Out-of-range
+  // buffer offsets read 0: nothing past the end of x or the scale array is
+  // touched.
   const bool vec_scales = (p.NW % 8) == 0 && (reinterpret_cast<uintptr_t>(p.scale) & 15u) == 0;
   u32x4_t sv[SPT];
   {
@@ -191,28 +177,12 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
     const uint32_t sbytes = (uint32_t)((uint64_t)((p.K + p.gs - 1) / p.gs) * p.N * 2u);
     const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(p.scale), (short)0, (int)sbytes, 0x00020000);
-    const int u = tid % CPR, mb = tid / CPR;
-    u32x4_t xv[XPT];
-#pragma unroll
-    for (int k = 0; k < XPT; ++k) {
-      if constexpr (AG) break;
-      const int m = mb + k * (NT / CPR);
-      const uint32_t off =
-          (m < p.M && 8 * u < R) ? (uint32_t)(((int64_t)m * p.ldx + row0 + 8 * u) * 2) : 0x80000000u;
-      xv[k] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)off, 0, 0));
-    }
-    if constexpr (!AG) {
-#pragma unroll
-      for (int k = 0; k < XPT; ++k) {
-        const int m = mb + k * (NT / CPR);
-        *reinterpret_cast<u32x4_t*>(&s_x[m * XS + 8 * u]) = xv[k];
-      }
-    }
     // the block's statistic: thread t takes K chunk u0 = t % U (8 rows of K)
-    // for batch rows t / U, t / U + S, ... (U = R / 8 <= NT chunks, S = NT / U
-    // slices), 8 loads at a time
-    if (AG && own_sigma) {
-      const int U = R >> 3, S = NT / U;
+    // for batch rows t / U, t / U + S, ... (U = R / 8 <= NT chunks, S slices),
+    // 8 loads at a time, and leaves its maxima in LDS; whoever grades a row
+    // takes the maximum over the slices
+    if (own_sigma) {
+      const int U = R >> 3, S = sig_slices;
       const int u0 = tid % U, sl = tid / U;
       if (sl < S) {
         float mx[8];
@@ -227,77 +197,83 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
             v[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)off, 0, 0));
           }
 #pragma unroll
-          for (int i = 0; i < 8; ++i)
+          for (int i = 0; i < 8; ++i) {
+            if (i == 2 && m0 - sl + 2 * S >= p.M) break;  // block-uniform: no rows in the rest
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               mx[2 * e] = fmaxf(mx[2 * e], fabsf(to_f32<DT>((uint16_t)(v[i][e] & 0xFFFFu))));
               mx[2 * e + 1] = fmaxf(mx[2 * e + 1], fabsf(to_f32<DT>((uint16_t)(v[i][e] >> 16))));
             }
+          }
         }
-#pragma unroll
-        for (int e = 0; e < 8; ++e) sig_part[e] = mx[e];
-        sig_chunk = u0;
+        f32x4_t* dst = reinterpret_cast<f32x4_t*>(&s_sig[sl * R + 8 * u0]);
+        dst[0] = f32x4_t{mx[0], mx[1], mx[2], mx[3]};
+        dst[1] = f32x4_t{mx[4], mx[5], mx[6], mx[7]};
       }
     }
 #pragma unroll
     for (int k = 0; k < SPT; ++k) {
       const int h = tid + NT * k;  // (group, tile, half) chunk
-      const int gl = h >> 5, r = (h >> 1) & 15, hf = h & 1;
+      const int gl = h / (32 * CG), r = (h / (2 * CG)) & 15, hf = h % (2 * CG);
       const uint32_t off =
           (gl < n_groups && vec_scales)
               ? (uint32_t)(((int64_t)(g_first + gl) * p.N + (int64_t)r * p.NW + w0 + 8 * hf) * 2)
               : 0x80000000u;
       sv[k] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, (int)off, 0, 0));
     }
+    // more groups than those (short groups, long K ranges): stored at once
+    for (int h = tid + NT * SPT; h < n_groups * 32 * CG && vec_scales; h += NT) {
+      const int gl = h / (32 * CG), r = (h / (2 * CG)) & 15, hf = h % (2 * CG);
+      const uint32_t off = (uint32_t)(((int64_t)(g_first + gl) * p.N + (int64_t)r * p.NW + w0 + 8 * hf) * 2);
+      const u32x4_t v = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, (int)off, 0, 0));
+      *reinterpret_cast<u32x4_t*>(&s_scale[8 * h]) = v;
+      if constexpr (GUARD) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) smax = max(smax, max(v[e] & 0x7FFFu, (v[e] >> 16) & 0x7FFFu));
+      }
+    }
   }
   __syncthreads();
 
-  if (AG && own_sigma) {
-    if (sig_chunk >= 0) {
+  // ---- phase 1b (graded): grade each row: zone bits, correction-column value
+  // and zone-0 flip.  Rows with zone 0 active are consumed in offset binary
+  // (zone 0's digits flipped, u = int8(U & mask) + 128, and the column value
+  // removes the 128); other rows have bit 7 clear and need no flip:
+  //   w_eff * 2^sh = u + beta * 2^sh - (zone 0 active ? 128 : 0).
+  // A row with no active zone therefore contributes exact zeros.  Dense, every
+  // row has the same constants.
+  auto row_value = [&](uint32_t bits, int beta) -> uint16_t {
+    if constexpr (SC)  // -c_row of the scaled weight (u >> sh) - c_row, an exact fp16 integer
+      return f32_to_f16_bits(-(float)(1024 + ((bits & 1u) ? (128 >> SH) : 0) - beta));
+    else
+      return BOperand<DT>::correction(beta * (1 << SH) - ((bits & 1u) ? 128 : 0));
+  };
+  if constexpr (!DENSE) {
+    // (the loop that reads the caller's statistic from global memory is kept
+    // apart, so that the other has no global load and the scale loads stay in
+    // flight through it)
+    auto grade_row = [&](int rr, float s) {
+      const uint32_t bits = zone_bits<Z>(s, p.thr.t);
+      s_bv[rr] = row_value(bits, midpoint_bias<Z>(bits));
+      s_zb[rr] = (uint8_t)bits;
+    };
+    if (own_sigma) {  // this block's share of the batch statistic
+      for (int rr = tid; rr < R; rr += NT) {
+        float sg = 0.f;
+        for (int s0 = 0; s0 < sig_slices; s0 += 8) {  // eight reads in flight (past the last slice: that one again)
+          float v[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (sig_part[e] > 0.f) atomicMax(&s_sig[8 * sig_chunk + e], __float_as_uint(sig_part[e]));
+          for (int i = 0; i < 8; ++i) v[i] = s_sig[min(s0 + i, sig_slices - 1) * R + rr];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) sg = fmaxf(sg, v[i]);
+        }
+        grade_row(rr, sg);
+      }
+    } else {  // the batch statistic given by the caller
+      for (int rr = tid; rr < R; rr += NT) grade_row(rr, precomputed_sigma(p, row0 + rr));
     }
     __syncthreads();
   }
-
-  // ---- phase 1b: grade each row: correction-column value, zone-0 flip and
-  // plane offsets.  Rows with zone 0 active are consumed in offset binary (zone
-  // 0's digits flipped, u = int8(U & mask) + 128, and the column value removes
-  // the 128); other rows have bit 7 clear and need no flip:
-  //   w_eff * 2^sh = u + beta * 2^sh - (zone 0 active ? 128 : 0).
-  // A row with no active zone therefore contributes exact zeros.
-  // (the loop that reads the caller's statistic from global memory is kept
-  // apart, so that the others have no global load and the scale loads stay in
-  // flight through them)
-  auto grade_row = [&](int rr, float s) {
-    uint32_t bits = (1u << Z) - 1u;
-    if constexpr (!DENSE) bits = zone_bits<Z>(s, p.thr.t);
-    const int beta = DENSE ? 0 : midpoint_bias<Z>(bits);
-    if constexpr (SC)  // -c_row of the scaled weight (u >> sh) - c_row, an exact fp16 integer
-      s_bv[rr] = f32_to_f16_bits(-(float)(1024 + ((bits & 1u) ? (128 >> SH) : 0) - beta));
-    else
-      s_bv[rr] = BOperand<DT>::correction(beta * (1 << SH) - ((bits & 1u) ? 128 : 0));
-    s_xm[rr] = zone0_flip(bits);
-    const uint32_t row_bytes = (uint32_t)(row0 + rr) * (uint32_t)(Z * p.NW) * 4u;
-#pragma unroll
-    for (int z = 0; z < Z; ++z)
-      s_off[rr * Z + z] = ((bits >> z) & 1u) ? row_bytes + (uint32_t)z * (uint32_t)p.NW * 4u : 0x80000000u;
-  };
-  if (DENSE) {
-    for (int rr = tid; rr < R; rr += NT) grade_row(rr, 0.f);
-  } else if (AG && own_sigma) {  // this block's share of the batch statistic
-    for (int rr = tid; rr < R; rr += NT) grade_row(rr, __uint_as_float(s_sig[rr]));
-  } else if (AG || p.sigma != nullptr) {  // the batch statistic given by the caller
-    for (int rr = tid; rr < R; rr += NT) grade_row(rr, precomputed_sigma(p, row0 + rr));
-  } else {  // from the staged x
-    for (int rr = tid; rr < R; rr += NT) {
-      float s = fabsf(to_f32<DT>(s_x[rr]));
-      for (int m = 1; m < p.M; ++m) s = fmaxf(s, fabsf(to_f32<DT>(s_x[m * XS + rr])));
-      grade_row(rr, s);
-    }
-  }
-  __syncthreads();
 
   int up_exp = 0;  // the block's sums are scaled by 2^up_exp at the end
   // The scales into LDS, once the first tiles' plane loads are issued; then
@@ -310,18 +286,17 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
 #pragma unroll
       for (int k = 0; k < SPT; ++k) {
         const int h = tid + NT * k;
-        if ((h >> 5) < SC_GROUPS)
-          *reinterpret_cast<u32x4_t*>(&s_scale[(h >> 5) * 256 + ((h >> 1) & 15) * 16 + 8 * (h & 1)]) = sv[k];
+        if (h < SC_GROUPS * 32 * CG) *reinterpret_cast<u32x4_t*>(&s_scale[8 * h]) = sv[k];
         if constexpr (GUARD) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) smax = max(smax, max(sv[k][e] & 0x7FFFu, (sv[k][e] >> 16) & 0x7FFFu));
         }
       }
     } else {  // column count not a multiple of 128: element-wise scale staging
-      for (int idx = tid; idx < n_groups * 256; idx += NT) {
-        const int gl = idx >> 8, col = idx & 255;
-        const int wcol = min(w0 + (col & 15), p.NW - 1);
-        s_scale[idx] = p.scale[(int64_t)(g_first + gl) * p.N + (int64_t)(col >> 4) * p.NW + wcol];
+      for (int idx = tid; idx < n_groups * 16 * WB; idx += NT) {
+        const int gl = idx / (16 * WB), col = idx % (16 * WB);
+        const int wcol = min(w0 + col % WB, p.NW - 1);
+        s_scale[idx] = p.scale[(int64_t)(g_first + gl) * p.N + (int64_t)(col / WB) * p.NW + wcol];
         if constexpr (GUARD) smax = max(smax, (uint32_t)s_scale[idx] & 0x7FFFu);
       }
     }
@@ -332,7 +307,7 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
       if (hm > kScaleLimit) {
         up_exp = (int)(hm >> 10) - (int)(kScaleLimit >> 10);
         const float down = __builtin_ldexpf(1.f, -up_exp);
-        for (int idx = tid; idx < n_groups * 256; idx += NT)
+        for (int idx = tid; idx < n_groups * 16 * WB; idx += NT)
           s_scale[idx] = from_f32<DT>(to_f32<DT>(s_scale[idx]) * down);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       }
@@ -352,167 +327,160 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
 
   // Lanes past the last word column read the last valid column instead (their
   // outputs are never stored), so every address below is in bounds.
-  const bool col_ok = (w0 + c) < p.NW;
-  const int wc = col_ok ? (w0 + c) : (p.NW - 1);
+  const int cw = 16 * cg + c;  // this lane's word column in the block
+  const bool col_ok = (w0 + cw) < p.NW;
+  const int wc = col_ok ? (w0 + cw) : (p.NW - 1);
   const float post = BOperand<DT>::kUnit / (float)(1 << SH);
   const int t_begin = (nt * kw) / KW, t_end = (nt * (kw + 1)) / KW;
   const int tiles_per_group = p.gs >> 5;
 
-  // Plane words come from raw buffer loads: a (row, plane) a lane does not
-  // need has offset bit 31 set, past the buffer end, which returns 0 without a
-  // memory access.  The main loop issues every load unconditionally; tiles past
-  // the end of the wave's range go through a descriptor of size 0, so every
-  // one of their loads returns 0 without touching memory.  Wait counts stay
-  // static and two prefetched tiles remain in flight.
-  const int plane_bytes = (int)((uint64_t)p.K * (uint32_t)(Z * p.NW) * 4u);
+  // Loads past the end of the sub-range go through a descriptor of size 0, and
+  // a (row, plane) the grading does not need has offset bit 31 set, past the
+  // buffer end: both leave zeros in LDS without a memory access.  Lanes past
+  // the last word column load the last valid words (never stored).
+  const uint32_t row_bytes = (uint32_t)(Z * p.NW) * 4u;
+  const int plane_bytes = (int)((uint64_t)p.K * row_bytes);
   const __amdgpu_buffer_rsrc_t prsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.planes), (short)0, plane_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t prsrc_none =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(p.planes), (short)0, 0, 0x00020000);
-  const uint32_t lane_off = (uint32_t)wc * 4u;
-
-  typedef uint32_t offz_t __attribute__((ext_vector_type(Z)));
-  // plane words of one tile (and, above 16 rows, its A operand)
-  struct Tile {
-    uint32_t D[8][Z];
-    u32x4_t A[AG && !XL ? MT : 1];
-  };
   const __amdgpu_buffer_rsrc_t xsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(p.x), (short)0, (int)((uint64_t)p.M * p.ldx * 2u), 0x00020000);
   const __amdgpu_buffer_rsrc_t xsrc_none =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.x), (short)0, 0, 0x00020000);
-  auto issue = [&](int t, Tile& T) {
-    const bool live = t < t_end;
-    const __amdgpu_buffer_rsrc_t rs = live ? prsrc : prsrc_none;
-    const int sb = (live ? t : t_begin) * 32 + 8 * q;
+  // this lane's row, zone and byte offset in a tile for each of the wave's loads
+  uint32_t loff[IPW];
+  int lrow[IPW], lzone[IPW];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      offz_t o;
-      if constexpr (Z == 1) {
-        o = s_off[sb + e];
-      } else {
-        o = *reinterpret_cast<const offz_t*>(&s_off[(sb + e) * Z]);
-      }
+  for (int i = 0; i < IPW; ++i) {
+    constexpr int G = WB / GB;  // pieces per (e, z, q)
+    const int L = (sw * IPW + i) * 64 + lane;
+    const int pair = L / (4 * G), rem = L % (4 * G), qq = rem / G;
+    const int word = ((rem % G) * GB) ^ (CG == 2 ? 16 * (qq & 1) : 0);
+    lrow[i] = 8 * qq + pair / Z;
+    lzone[i] = pair % Z;
+    loff[i] = (uint32_t)lrow[i] * row_bytes + (uint32_t)(lzone[i] * p.NW + min(w0 + word, p.NW - GB)) * 4u;
+  }
+  typedef __attribute__((address_space(3))) void* lds_t;
+  // this wave's share of tile t (plane words, and x[16*mt + c][rows 8q .. 8q+7]
+  // as fragments of 1 KiB, lane l's 16 bytes at byte 16 l; rows m >= M read 0)
+  struct Zones { uint32_t z[DENSE ? 1 : IPW]; };  // zone bits of the rows this lane loads (graded)
+  auto read_zones = [&](int t) {
+    Zones zn;
+    if constexpr (!DENSE) {
+      const int tt = t < t_end ? t : t_begin;
 #pragma unroll
-      for (int z = 0; z < Z; ++z) {
-        const uint32_t oz = (Z == 1) ? (uint32_t)o[0] : (uint32_t)o[z];
-        T.D[e][z] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)(oz + lane_off), 0, 0);
-      }
+      for (int i = 0; i < IPW; ++i) zn.z[i] = s_zb[tt * 32 + lrow[i]];
     }
-    if constexpr (AG && !XL) {  // x[16*mt + c][rows 8q .. 8q+7 of the tile]; rows m >= M read 0
-      const __amdgpu_buffer_rsrc_t xs = live ? xsrc : xsrc_none;
+    return zn;
+  };
+  auto load_tile = [&](int t, unsigned char* pl, unsigned char* xr, const Zones& zn) {
+    const bool live = t < t_end;
+    const int tt = live ? t : t_begin;
+    const __amdgpu_buffer_rsrc_t xs = live ? xsrc : xsrc_none;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int m = 16 * mt + c;
-        const uint32_t off = m < p.M ? (uint32_t)(((int64_t)m * p.ldx + row0 + sb) * 2) : 0x80000000u;
-        T.A[mt] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(xs, (int)off, 0, 0));
-      }
+    for (int h = 0; h < XPW; ++h) {
+      const int mt = XPW * sw + h;
+      if (MT % SG != 0 && mt >= MT) break;  // wave-uniform
+      const int m = 16 * mt + c;
+      const uint32_t off = m < p.M ? (uint32_t)(((int64_t)m * p.ldx + row0 + tt * 32 + 8 * q) * 2) : 0x80000000u;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xs, (lds_t)(xr + (kw * MT + mt) * 1024), 16, (int)off, 0, 0, 0);
+    }
+    const __amdgpu_buffer_rsrc_t rs = live ? prsrc : prsrc_none;
+    const int sbase = (int)((uint32_t)(row0 + tt * 32) * row_bytes);
+#pragma unroll
+    for (int i = 0; i < IPW; ++i) {
+      const int gi = sw * IPW + i;
+      if (IPT % SG != 0 && gi >= IPT) break;  // wave-uniform
+      uint32_t off = loff[i];
+      if constexpr (!DENSE) off = ((zn.z[i] >> lzone[i]) & 1u) ? off : 0x80000000u;
+      const lds_t dst = (lds_t)(pl + kw * TILE + gi * 64 * GB * 4);
+      if constexpr (WIDE)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 16, (int)off, sbase, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, (int)off, sbase, 0, 0);
     }
   };
+  // the LDS words this lane reads of a tile
+  const int dpos = kw * TILE + (q * WB + ((16 * cg) ^ (CG == 2 ? 16 * (q & 1) : 0)) + c) * 4;
 
-  // one tile: optional prefetch of tile t+2, unpack, MFMA, group epilogue
   // position of the current tile in its scale group and the group's index in
   // the staged scales, advanced per tile (no divisions in the loop)
   int gpos = (tile0 + t_begin) % tiles_per_group;
   int gloc = (tile0 + t_begin) / tiles_per_group - g_first;
   uint32_t s2[NJ][4];  // scaled path: (s, s) of the current group's columns
-  // this wave's share of x[16*mt + c][rows 8q .. 8q+7 of tile t] (fragments
-  // mt = XF jg .. XF jg + XF - 1) into slot xr: lane l's 16 bytes land at
-  // byte 16 l of the fragment's KiB; rows m >= M, and tiles past the range,
-  // read nothing (and are never used)
-  auto load_x_lds = [&](int t, unsigned char* xr) {
-    const __amdgpu_buffer_rsrc_t xs = t < t_end ? xsrc : xsrc_none;
-#pragma unroll
-    for (int h = 0; h < XF; ++h) {
-      const int mt = XF * jg + h;
-      const int m = 16 * mt + c;
-      const uint32_t off = m < p.M ? (uint32_t)(((int64_t)m * p.ldx + row0 + t * 32 + 8 * q) * 2) : 0x80000000u;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          xs, (__attribute__((address_space(3))) void*)(xr + (kw * MT + mt) * 1024), 16, (int)off, 0, 0, 0);
-    }
-  };
-  auto step = [&](int t, Tile& Tc, bool prefetch, Tile& Tn, unsigned char* xcur, unsigned char* xnext) {
+  const uint16_t dense_value = row_value((1u << Z) - 1u, 0);
+  // one tile: handshake, loads of tile t + PF, unpack, MFMA, group epilogue
+  auto step = [&](int t, const unsigned char* pcur, const unsigned char* xcur, unsigned char* pnext, unsigned char* xnext) {
     const bool first_of_group = (t == t_begin) || (gpos == 0);
     const bool last_of_group = (t + 1 == t_end) || (gpos + 1 == tiles_per_group);
     const int sb = t * 32 + 8 * q;
 
-    // A operand: x[16*mt + c][rows 8q .. 8q+7 of the tile].  At 17-64 rows
-    // it is read from the K sub-range's LDS slot, filled in shares by its
-    // waves one tile ahead (loaded before the next tile's plane words: memory
-    // operations complete in order, so waiting for it leaves those in
-    // flight).
-    u32x4_t A[MT];
-    auto load_a = [&]() {
+    // own share of tile t: wait until at most the loads issued after it are in
+    // flight (every wave's share of them, at least).  Then the handshake:
+    // publish it, and wait until every other wave of the K sub-range has
+    // published its share, which also means it has read the slots of earlier
+    // tiles, the one the next loads overwrite among them.  Every wave
+    // publishes before it waits, so every wait ends (and is bounded: one that
+    // outlasted ~2^22 polls would end, with a wrong tile, rather than hang).
+    const Zones zn = read_zones(t + PF);
+    constexpr int LATER = (PF - 1) * ((IPT % SG == 0 ? IPW : 0) + (MT % SG == 0 ? XPW : 0));
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory");
+    if (lane == 0) __hip_atomic_store(&s_flag[wave], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        if constexpr (AG) {
-          A[mt] = Tc.A[mt];
-        } else {
-          A[mt] = *reinterpret_cast<const u32x4_t*>(&s_x[(16 * mt + c) * XS + sb]);
-        }
+    for (int pj = 0; pj < SG; ++pj) {
+      if (pj == sw) continue;
+      for (int spin = 0; spin < (1 << 22) &&
+                         __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                             &s_flag[kw * SG + pj], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < t;
+           ++spin) {
       }
-    };
-    if constexpr (XL) {
-      // own share of tile t (its loads waited for by the compiler), then the
-      // handshake: publish it, and wait until every other wave of the K
-      // sub-range has published its share, which also means it has read the
-      // slots of earlier tiles, the one the next loads overwrite among them.
-      // Every wave publishes before it waits, so every wait ends.
-      const unsigned char* xb = xcur + kw * MT * 1024 + lane * 16;
-      // one dword of the own share read back: the compiler waits for this
-      // wave's loads into the slot before it
-      const uint32_t probe = *reinterpret_cast<const uint32_t*>(xb + XF * jg * 1024);
-      asm volatile("" ::"v"(probe));
-      if (lane == 0) __hip_atomic_store(&s_xflag[wave], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      // (bounded: a wait that outlasted ~2^20 sleeps would end, with a wrong
-      // tile, rather than hang; the others publish within microseconds)
-#pragma unroll
-      for (int pj = 0; pj < JG; ++pj) {
-        if (pj == jg) continue;
-        for (int spin = 0; spin < (1 << 20) &&
-                           __builtin_amdgcn_readfirstlane(__hip_atomic_load(
-                               &s_xflag[kw * JG + pj], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < t;
-             ++spin)
-          __builtin_amdgcn_s_sleep(1);
-      }
-      // (always: a tile past the range reads nothing; at 17-32 rows the last
-      // two steps take no plane prefetch but the second still needs its x)
-      load_x_lds(t + 1, xnext);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) A[mt] = *reinterpret_cast<const u32x4_t*>(xb + mt * 1024);
     }
-    if (prefetch) issue(t + PF, Tn);
+    asm volatile("" ::: "memory");
+    load_tile(t + PF, pnext, xnext, zn);
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (!XL) load_a();
 
-    const u32x4_t bv = *reinterpret_cast<const u32x4_t*>(&s_bv[sb]);
+    u32x4_t A[MT];  // x[16*mt + c][rows 8q .. 8q+7 of the tile]
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      A[mt] = *reinterpret_cast<const u32x4_t*>(xcur + (kw * MT + mt) * 1024 + lane * 16);
+    uint32_t D[8][Z];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int z = 0; z < Z; ++z)
+        D[e][z] = *reinterpret_cast<const uint32_t*>(pcur + dpos + (e * Z + z) * 16 * WB);
 
     // Rebuild the code bytes (offset binary) and turn them into B operands.
+    u32x4_t bv;
     uint32_t xm[8];
-    {
-      const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(&s_xm[sb]);
-      const u32x4_t hi = *reinterpret_cast<const u32x4_t*>(&s_xm[sb + 4]);
+    if constexpr (DENSE) {
+      const uint32_t v = (uint32_t)dense_value * 0x00010001u;
+      bv = u32x4_t{v, v, v, v};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        xm[e] = lo[e];
-        xm[e + 4] = hi[e];
-      }
+      for (int e = 0; e < 8; ++e) xm[e] = 0xAAAAAAAAu;
+    } else {
+      bv = *reinterpret_cast<const u32x4_t*>(&s_bv[sb]);
+      const u32x2_t zb = *reinterpret_cast<const u32x2_t*>(&s_zb[sb]);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)  // zone 0's flip: bit 0 of the row's byte, spread
+        xm[e] = (uint32_t)((int32_t)(zb[e >> 2] << (31 - 8 * (e & 3))) >> 31) & 0xAAAAAAAAu;
     }
-    prepare_planes<Z>(Tc.D, xm);
+    prepare_planes<Z>(D, xm);
     if constexpr (SC) {
       // B = RNE(w * s) with s2 = (s, s) of this lane's columns for the group
       // and bv = (-c_row, -c_row') per row pair; the output accumulates directly.
       if (first_of_group) {
-        const uint16_t* srow = &s_scale[gloc * 256 + 64 * jg * NJ + c];
+        const uint16_t* srow = &s_scale[(gloc * 16 + 4 * jg * NJ) * WB + cw];
 #pragma unroll
         for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
-          for (int b = 0; b < 4; ++b) s2[jj][b] = (uint32_t)srow[(4 * jj + b) * 16] * 0x00010001u;
+          for (int b = 0; b < 4; ++b) s2[jj][b] = (uint32_t)srow[(4 * jj + b) * WB] * 0x00010001u;
       }
 #pragma unroll
       for (int jj = 0; jj < NJ; ++jj) {
         uint32_t V[8];
-        code_dwords<Z>(Tc.D, jg * NJ + jj, V);
+        code_dwords<Z>(D, jg * NJ + jj, V);
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
           u32x4_t B;
@@ -523,37 +491,41 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
         }
       }
     }
-#pragma unroll
-    for (int jj = 0; jj < (SC ? 0 : NJ); ++jj) {
-      const int j = jg * NJ + jj;
-      uint32_t V[8];
-      code_dwords<Z>(Tc.D, j, V);
-      u32x4_t B[4];
-      BOperand<DT>::build(V, B);
-      // the first tile of a scale group starts its sums from zero
+    if constexpr (!SC) {
       if (first_of_group) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int mt = 0; mt < MT; ++mt) {
+          Cv[mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) C[mt][jj][b] = mfma16x16x32<DT>(A[mt], B[b], f32x4_t{0.f, 0.f, 0.f, 0.f});
-      } else {
+          for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) C[mt][jj][b] = mfma16x16x32<DT>(A[mt], B[b], C[mt][jj][b]);
+            for (int b = 0; b < 4; ++b) C[mt][jj][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
       }
-    }
 #pragma unroll
-    for (int mt = 0; mt < (SC ? 0 : MT); ++mt)
-      Cv[mt] = mfma16x16x32<DT>(A[mt], bv, first_of_group ? f32x4_t{0.f, 0.f, 0.f, 0.f} : Cv[mt]);
+      for (int jj = 0; jj < NJ; ++jj) {
+        uint32_t V[8];
+        code_dwords<Z>(D, jg * NJ + jj, V);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          u32x4_t B;
+#pragma unroll
+          for (int pp = 0; pp < 4; ++pp) B[pp] = BOperand<DT>::pair(V[2 * pp], V[2 * pp + 1], b);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) C[mt][jj][b] = mfma16x16x32<DT>(A[mt], B, C[mt][jj][b]);
+        }
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) Cv[mt] = mfma16x16x32<DT>(A[mt], bv, Cv[mt]);
+    }
 
     if (!SC && last_of_group) {  // y += s[g][n] * 2^-sh * (C + Cv), scales from LDS
-      const uint16_t* srow = &s_scale[gloc * 256 + 64 * jg * NJ + c];
+      const uint16_t* srow = &s_scale[(gloc * 16 + 4 * jg * NJ) * WB + cw];
 #pragma unroll
       for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
-          const float sc = to_f32<DT>(srow[(4 * jj + b) * 16]) * post;
+          const float sc = to_f32<DT>(srow[(4 * jj + b) * WB]) * post;
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -569,37 +541,40 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
   };
 
   {
-    Tile TA, TB, TC;
     int t = t_begin;
+    load_tile(t_begin, s_pl0, s_xr0, read_zones(t_begin));
     if constexpr (PF == 2) {
-      // three tile buffers: tiles t+1 and t+2 are in flight while tile t is
-      // unpacked; the first x tile before the first plane words, as in every
-      // step
-      if constexpr (XL) load_x_lds(t_begin, s_xr0);
-      issue(t_begin, TA);
-      issue(t_begin + 1, TB);
+      load_tile(t_begin + 1, s_pl1, s_xr1, read_zones(t_begin + 1));
       stage_scales();
-      for (; t + 3 <= t_end; t += 3) {
-        step(t, TA, true, TC, s_xr0, s_xr1);
-        step(t + 1, TB, true, TA, s_xr1, s_xr2);
-        step(t + 2, TC, true, TB, s_xr2, s_xr0);
+if constexpr (MT == 1) {
+        for (; t + 3 <= t_end; t += 3) {
+          step(t, s_pl0, s_xr0, s_pl2, s_xr2);
+          step(t + 1, s_pl1, s_xr1, s_pl0, s_xr0);
+          step(t + 2, s_pl2, s_xr2, s_pl1, s_xr1);
+        }
+        if (t < t_end) step(t, s_pl0, s_xr0, s_pl2, s_xr2);
+        if (t + 1 < t_end) step(t + 1, s_pl1, s_xr1, s_pl0, s_xr0);
+      } else {  // (one copy per slot: 1-2 % faster here, 2-4 % slower at 5-16 rows)
+        for (; t < t_end; t += 3) {
+          step(t, s_pl0, s_xr0, s_pl2, s_xr2);
+          if (t + 1 >= t_end) break;
+          step(t + 1, s_pl1, s_xr1, s_pl0, s_xr0);
+          if (t + 2 >= t_end) break;
+          step(t + 2, s_pl2, s_xr2, s_pl1, s_xr1);
+        }
       }
-      // at most two tiles left, already loaded into TA and TB
-      if (t < t_end) step(t, TA, false, TC, s_xr0, s_xr1);
-      if (t + 1 < t_end) step(t + 1, TB, false, TC, s_xr1, s_xr2);
     } else {
-      // two tile buffers: tile t+1 is in flight while tile t is unpacked
-      // the first x tile before the first plane words, as in every step
-      if constexpr (XL) load_x_lds(t_begin, s_xr0);
-      issue(t_begin, TA);
       stage_scales();
-      for (; t + 2 <= t_end; t += 2) {
-        step(t, TA, true, TB, s_xr0, s_xr1);
-        step(t + 1, TB, true, TA, s_xr1, s_xr0);
+      for (; t < t_end; t += 2) {
+        step(t, s_pl0, s_xr0, s_pl1, s_xr1);
+        if (t + 1 >= t_end) break;
+        step(t + 1, s_pl1, s_xr1, s_pl0, s_xr0);
       }
-      if (t < t_end) step(t, TA, false, TB, s_xr0, s_xr1);
     }
   }
+  // the slots are reused below: none of this wave's loads may still be on its
+  // way to them (loads past the range leave zeros)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   if (GUARD && up_exp > 0) {
     const float up = __builtin_ldexpf(1.f, up_exp);
@@ -621,13 +596,16 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
   // leave their sums in the staging area, free now, one slot per wave.
   auto owns = [&](int mt) { return kw == mt % KW; };  // wave-uniform
   if (KW > 1) {
-    constexpr int SLOT = NJ * 4 * 64;  // f32x4 per wave slot
+    auto red_slot = [&](int i) -> f32x4_t* {  // wave slots are spread over the plane slots
+      unsigned char* base = i < RED_PER ? s_pl0 : (PF == 1 || i < 2 * RED_PER) ? s_pl1 : s_pl2;
+      return reinterpret_cast<f32x4_t*>(base + (i % RED_PER) * RED_SLOT);
+    };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int own = mt % KW;
       __syncthreads();
       if (kw != own) {
-        f32x4_t* slot = s_red + ((kw < own ? kw : kw - 1) * JG + jg) * SLOT;
+        f32x4_t* slot = red_slot((kw < own ? kw : kw - 1) * SG + sw);
 #pragma unroll
         for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
@@ -641,7 +619,7 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
           for (int b = 0; b < 4; ++b) {
             auto part = [&](int k2) -> f32x4_t {  // sub-range k2's sums
               if (k2 == own) return Y[mt][jj][b];
-              return s_red[((k2 < own ? k2 : k2 - 1) * JG + jg) * SLOT + (jj * 4 + b) * 64 + lane];
+              return red_slot((k2 < own ? k2 : k2 - 1) * SG + sw)[(jj * 4 + b) * 64 + lane];
             };
             f32x4_t acc = part(0);
 #pragma unroll
@@ -740,7 +718,7 @@ __global__ __launch_bounds__((64 * decode_waves<DT, MT>()), 1) void decode_kerne
           }
     }
   }
-  if (p.counters != nullptr) splitk_complete<DT, 4 * MT * 256 / NT, NT>(p, lb % col_blocks, w0, 16);
+  if (p.counters != nullptr) splitk_complete<DT, 1024 * MT * CG / NT, NT>(p, lb % col_blocks, w0, WB);
 }
 
 // y[m][n] = cast(sum_{s=0..splits-1} partial[s][m][n]) (+ bias), four
@@ -820,27 +798,43 @@ __global__ __launch_bounds__(256) void sigma_kernel(const uint16_t* __restrict__
   }
 }
 
-DecodePlan plan_decode(int64_t M, int64_t K, int64_t N) {
+DecodePlan plan_decode(int64_t M, int64_t K, int64_t N, int max_bits, bool dense, bool wide) {
   DecodePlan pl{};
+  pl.wide = wide;
   pl.mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-  const int64_t NW = N / 16;
-  pl.col_blocks = (int)((NW + 15) / 16);
-  const int64_t T = K / 32;
-  const int kw = pl.mt == 4 ? 4 : 4 / pl.mt;  // K sub-ranges per block (four on the scaled path)
-  const int64_t tiles_max = (pl.mt >= 2 ? kDecodeRowsPerBlock : kDecodeRowsPerBlock / pl.mt) / 32;
-  const int64_t min_splits = (T + tiles_max - 1) / tiles_max;
-  // one block per CU, all blocks resident at once: the per-block set-up
-  // (staging, grading) is paid once per CU rather than once per round
-  const int64_t want = kTargetBlocks / pl.col_blocks > 0 ? kTargetBlocks / pl.col_blocks : 1;
-  int64_t max_splits = T / (2 * kw);
-  if (max_splits < 1) max_splits = 1;
-  int64_t splits = want < max_splits ? want : max_splits;
-  if (splits < min_splits) splits = min_splits;
+  const int64_t NW = N / 16, T = K / 32;
   const int64_t bytes_per_split = M * N * (int64_t)sizeof(float);
-  if (splits > 1 && bytes_per_split > 0) {
-    int64_t cap = (int64_t)kMaxPartialBytes / bytes_per_split;
-    if (cap < min_splits) cap = min_splits;
-    if (splits > cap) splits = cap;
+  int64_t splits = 1;
+  auto choose = [&](int cg) {
+    pl.cg = cg;
+    pl.col_blocks = (int)((NW + 16 * cg - 1) / (16 * cg));
+    const int kw = 4 / cg;  // K sub-ranges per block (at most)
+    const int64_t tiles_max = decode_rows_per_block(cg) / 32;
+    const int64_t min_splits = (T + tiles_max - 1) / tiles_max;
+    // one block per CU, all blocks resident at once: the per-block set-up
+    // (staging, grading) is paid once per CU rather than once per round
+    const int64_t want = kTargetBlocks / pl.col_blocks > 0 ? kTargetBlocks / pl.col_blocks : 1;
+    int64_t max_splits = T / (2 * kw);
+    if (max_splits < 1) max_splits = 1;
+    splits = want < max_splits ? want : max_splits;
+    if (splits < min_splits) splits = min_splits;
+    if (splits > 1 && bytes_per_split > 0) {
+      int64_t cap = (int64_t)kMaxPartialBytes / bytes_per_split;
+      if (cap < min_splits) cap = min_splits;
+      if (splits > cap) splits = cap;
+    }
+  };
+  // Dense batches of up to 32 rows are bound by the plane traffic, which
+  // blocks of 32 word columns read in whole 128-byte lines, for twice the K
+  // ranges and so twice the partial sums: taken where those stay below 0.3 of
+  // the plane bytes (16 rows, 16 / 32 columns: gate_up 46 / 36 us, down 25.8 /
+  // 23.0, Llama-3-70B gate_up 147 / 126; 24 rows gate_up 49 / 42; above the
+  // line qkv 16.4 / 16.9, o_proj 14.1 / 15.5).  Graded batches read fewer
+  // planes and are bound by their unpacking (gate_up 29.9 / 33.5 us).
+  choose(1);
+  if (wide && dense && pl.mt <= 2) {
+    choose(2);
+    if (splits * 16 * pl.mt * 4 * 10 > 3 * K * max_bits / 8) choose(1);
   }
   if (splits < 1) splits = 1;
   int64_t tps = (T + splits - 1) / splits;
@@ -855,12 +849,12 @@ DecodePlan plan_decode(int64_t M, int64_t K, int64_t N) {
 
 template <typename DT, int MT, int Z>
 static void launch_decode_t(const DecodeParams& p, const DecodePlan& pl, bool dense, hipStream_t st) {
-  const dim3 grid(pl.col_blocks * pl.splits);
-  const dim3 block(64 * decode_waves<DT, MT>());
-  if (dense)
-    launch_main_kernel(decode_kernel<DT, MT, Z, true>, grid, block, st, p);
-  else
-    launch_main_kernel(decode_kernel<DT, MT, Z, false>, grid, block, st, p);
+  const dim3 grid(pl.col_blocks * pl.splits), block(64 * kDecodeWaves);
+  auto kernel = dense ? decode_kernel<DT, MT, Z, true, false, 1> : decode_kernel<DT, MT, Z, false, false, 1>;
+  if (pl.wide) kernel = dense ? decode_kernel<DT, MT, Z, true, true, 1> : decode_kernel<DT, MT, Z, false, true, 1>;
+  if constexpr (MT <= 2)
+    if (pl.cg == 2) kernel = decode_kernel<DT, MT, Z, true, true, 2>;  // (dense only: plan_decode)
+  launch_main_kernel(kernel, grid, block, st, p);
 }
 
 template <typename DT, int MT>

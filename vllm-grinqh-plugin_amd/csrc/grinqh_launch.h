@@ -39,13 +39,16 @@ struct DecodeParams {
 
 struct DecodePlan {
   int mt;      // 16-row m-tiles: 1, 2 or 4 (M <= 16, 32, 64)
+  int cg;      // decode kernel: groups of 16 word columns per block
+  bool wide;   // decode kernel: 16-byte plane loads
   int splits;
   int tiles_per_split;
   int col_blocks;
   size_t workspace;  // partial-sum bytes, 0 if splits == 1
 };
 
-DecodePlan plan_decode(int64_t M, int64_t K, int64_t N);
+// wide: plane rows are 16-byte aligned (N % 64 == 0 and an aligned array)
+DecodePlan plan_decode(int64_t M, int64_t K, int64_t N, int max_bits, bool dense, bool wide);
 
 // Split-K completion counters (one per column block) at the start of the
 // workspace; larger column counts fall back to the reduce kernel.
