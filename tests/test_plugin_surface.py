@@ -193,3 +193,24 @@ def test_gpu_steps_refuse_cpu_tensors(gq):
     layer.grinqh_use_marlin = False
     with pytest.raises(ValueError, match="no CPU path"):
         method.apply(layer, torch.zeros(1, 256, dtype=torch.float16))
+
+
+def test_op_registration_layers():
+    """The op's device kernel sits below the custom op's registration: host
+    tensors are refused, fake tensors give the shape, and a backward raises."""
+    import grinqh.kernel  # noqa: F401
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    op = torch.ops.grinqh.gemm_or_gemv
+    x, P, s = torch.zeros(2, 128), torch.zeros(128, 16, dtype=torch.int32), torch.zeros(1, 64)
+    with pytest.raises(ValueError, match="HIP device"):
+        op(x, P, s, None, 8, 128, 16, [0.0] * 4)
+    assert torch._C._dispatch_has_kernel_for_dispatch_key("grinqh::gemm_or_gemv", "CUDA")
+    with FakeTensorMode():
+        y = op(torch.empty(3, 5, 128, device="cuda"), torch.empty(128, 16, dtype=torch.int32, device="cuda"),
+               torch.empty(1, 64, device="cuda"), None, 8, 128, 16, [0.0] * 4)
+        assert tuple(y.shape) == (3, 5, 64) and y.device.type == "cuda"
+    x = torch.empty(3, 128, device="meta", requires_grad=True)
+    z = op(x, torch.empty(128, 16, dtype=torch.int32, device="meta"), torch.empty(1, 64, device="meta"), None, 8, 128,
+           16, [0.0] * 4)
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        z.sum().backward()

@@ -127,7 +127,7 @@ def run_product(x: torch.Tensor, weight_packed: torch.Tensor, weight_scale: torc
     dt = _dtype_code(x.dtype)
     K = x.shape[-1]
     N = 4 * int(original_n)
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
     if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
         x2 = x2.contiguous()
     M = x2.shape[0]
@@ -152,7 +152,7 @@ def run_product(x: torch.Tensor, weight_packed: torch.Tensor, weight_scale: torc
     y = torch.empty((M, N), dtype=x.dtype, device=x.device)
     lib = _lib.load_library()
     mode_code = _MODES[mode]
-    stream = torch.cuda.current_stream(x.device).cuda_stream
+    stream = torch._C._cuda_getCurrentRawStream(x.device.index)  # current_stream() without its wrapper object
     nbytes = lib.grinqh_workspace_bytes(M, K, N, max_bits, mode_code)
     ws = _WORKSPACES.get(x.device, stream, nbytes)
     _lib.check(lib.grinqh_gemm_or_gemv(
@@ -160,7 +160,7 @@ def run_product(x: torch.Tensor, weight_packed: torch.Tensor, weight_scale: torc
         max_bits, group_size, _lib.thresholds_f32(thresholds), mode_code,
         ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, stream),
         "grinqh_gemm_or_gemv")
-    return y.view(*x.shape[:-1], N)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 
 @torch.library.custom_op("grinqh::gemm_or_gemv", mutates_args=())
@@ -183,6 +183,21 @@ def grinqh_gemm_or_gemv(
 @grinqh_gemm_or_gemv.register_fake
 def _fake(x, weight_packed, weight_scale, bias, max_bits, group_size, original_n, thresholds, use_marlin=False):
     return torch.empty(x.shape[:-1] + (original_n * 4,), device=x.device, dtype=x.dtype)
+
+
+def _gemm_or_gemv_device(x, weight_packed, weight_scale, bias, max_bits, group_size, original_n, thresholds,
+                         use_marlin=False):
+    return run_product(x, weight_packed, weight_scale, bias, max_bits, group_size, original_n, thresholds,
+                       _BATCH_GRADING)
+
+
+# The op's kernel for device tensors, registered below the custom op's own
+# wrapper, which compares the storages of every argument and result on each
+# call (the result here is always a new tensor): 3.5 us of a call's 15 us of
+# dispatch.  Autograd, fake tensors and tracing stay the custom op's; host
+# tensors reach it and are refused there.
+_DEVICE_KERNEL = torch.library.Library("grinqh", "FRAGMENT")
+_DEVICE_KERNEL.impl("gemm_or_gemv", _gemm_or_gemv_device, "CUDA")
 
 
 def grinqh_gemv_batch_union(x: torch.Tensor, weight_packed: torch.Tensor, weight_scale: torch.Tensor,
