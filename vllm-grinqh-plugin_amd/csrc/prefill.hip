@@ -49,7 +49,7 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void prefill_kernel(PrefillParams 
   constexpr int AL = BM * CPR / NP;
   constexpr int RPT = BK / 16;      // rows per dequantizing thread
   constexpr int JPT = 4 * 256 / NP; // output dwords j per dequantizing thread
-  static_assert(!WS || (WAVES == 8 && PD == 2), "warp-specialised shape");
+  static_assert(!WS || (WAVES == 8 && PD % 2 == 0), "warp-specialised shape");
   static_assert(MTW >= 1 && AL >= 1 && RPT % 2 == 0 && JPT >= 1, "tile shape");
 
   __shared__ __align__(16) uint16_t s_a[2][BM * KP];
@@ -267,32 +267,36 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void prefill_kernel(PrefillParams 
   // conditional store made it wait for every outstanding load, scale loads
   // included, at the top of each stage).  Stage t is multiplied from LDS
   // buffer (t - s_begin) & 1.
-  Slot LA, LB;
   int s = s_begin;
   if constexpr (WS) {
     // Both roles pass the same number of barriers: one after the first
-    // stage is stored, then one per stage but the last.  Stage t lives in
-    // LDS buffer (t - s_begin) & 1 and in register slot (t - s_begin) & 1
-    // (LA even, LB odd); two stages of loads are in flight.  Loads past the
-    // range repeat its last stage (unconditional loads keep the wait counts
-    // exact) and are never stored.
+    // stage is stored, then one per stage but the last.  Stage t (from 0) lives
+    // in LDS buffer t & 1 and in register slot t % PD; PD stages of loads are
+    // in flight.  Loads past the range repeat its last stage (unconditional
+    // loads keep the wait counts exact) and are never stored.  All PD stages
+    // are issued before the first is stored; four instead of two stages in
+    // flight were slower (four linears at 150 rows: 192.3 against 189.7 us).
     if (wave < NP / 64) {
-      const int last = s_end - 1;
-      load_stage(s_begin, LA);
-      store_stage(0, LA);
-      load_stage(min(s_begin + 1, last), LB);
-      load_stage(min(s_begin + 2, last), LA);
+      const int n = s_end - s_begin, last = s_end - 1;
+      Slot L[PD];
+#pragma unroll
+      for (int i = 0; i < PD; ++i) load_stage(min(s_begin + i, last), L[i]);
+      store_stage(0, L[0]);
+      load_stage(min(s_begin + PD, last), L[0]);
       __syncthreads();
-      for (; s + 2 < s_end; s += 2) {  // store stages s+1 and s+2
-        store_stage(1, LB);
-        load_stage(min(s + 3, last), LB);
-        __syncthreads();
-        store_stage(0, LA);
-        load_stage(min(s + 4, last), LA);
-        __syncthreads();
+      int t = 1;
+      for (; t + PD <= n; t += PD) {
+#pragma unroll
+        for (int i = 0; i < PD; ++i) {
+          store_stage((1 + i) & 1, L[(1 + i) % PD]);
+          load_stage(min(s_begin + t + i + PD, last), L[(1 + i) % PD]);
+          __syncthreads();
+        }
       }
-      if (s + 1 < s_end) {  // store stage s+1
-        store_stage(1, LB);
+#pragma unroll
+      for (int i = 0; i < PD - 1; ++i) {  // the stages left, loaded already
+        if (t + i >= n) break;
+        store_stage((1 + i) & 1, L[(1 + i) % PD]);
         __syncthreads();
       }
       return;  // the multiplying waves write the output
@@ -304,6 +308,7 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void prefill_kernel(PrefillParams 
     }
     multiply_stage((s - s_begin) & 1);
   } else if constexpr (PD == 1) {
+    Slot LA;
     load_stage(s_begin, LA);
     store_stage(0, LA);
     __syncthreads();
@@ -319,6 +324,7 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void prefill_kernel(PrefillParams 
     // two stages in flight: at the top of each iteration stage s is in LDS
     // buffer 0 and stage s+1 is loading into LB (a single-stage range loads
     // its stage twice, harmlessly)
+    Slot LA, LB;
     load_stage(s_begin, LA);
     store_stage(0, LA);
     load_stage(s + 1 < s_end ? s + 1 : s, LB);
@@ -354,6 +360,36 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void prefill_kernel(PrefillParams 
 
   // epilogue: lane (c, q) holds rows 4q..4q+3 of each 16 x 16 tile
   const bool col_ok = (w0 + c) < p.NW;
+  // Partial sums of a K range (kMaxPrefillPartialBytes at most, so 32-bit
+  // offsets do): buffer stores without branches; a row or column past the
+  // output has its offset past the range's slab, where the store is dropped.
+  // With a bounds branch around each of a lane's up to 128 stores the output
+  // took about 4 us of a launch: 150 rows, dense fp16, qkv 33.8 -> 29.8 us,
+  // o_proj 25.0 -> 21.6, down 57.2 -> 52 (kernel times on one MI355X).
+  if (p.splits > 1) {
+    const __amdgpu_buffer_rsrc_t prs =
+        __builtin_amdgcn_make_buffer_rsrc(p.partial + (int64_t)blockIdx.z * p.M * p.N, (short)0,
+                                          (int)((uint32_t)p.M * (uint32_t)p.N * 4u), 0x00020000);
+#pragma unroll
+    for (int i = 0; i < MTW; ++i) {
+      uint32_t roff[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + wm * WM + 16 * i + 4 * q + e;
+        roff[e] = (m < p.M && col_ok) ? ((uint32_t)m * (uint32_t)p.N + (uint32_t)(w0 + c)) * 4u : 0x80000000u;
+      }
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const uint32_t coff = (uint32_t)(8 * wn + r) * (uint32_t)p.NW * 4u;  // wave-uniform
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = DENSE ? acc[i][r][e] : graded_nonfinite_to_nan(GUARD ? acc[i][r][e] * up_scale : acc[i][r][e]);
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), prs, (int)roff[e], (int)coff, 0);
+        }
+      }
+    }
+    return;
+  }
   if (!col_ok) return;
 #pragma unroll
   for (int i = 0; i < MTW; ++i)
@@ -365,10 +401,7 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void prefill_kernel(PrefillParams 
         const int m = m0 + wm * WM + 16 * i + 4 * q + e;
         if (m >= p.M) continue;
         const float v = DENSE ? acc[i][r][e] : graded_nonfinite_to_nan(GUARD ? acc[i][r][e] * up_scale : acc[i][r][e]);
-        if (p.splits == 1)
-          p.y[(int64_t)m * p.N + n] = finish_output<DT>(v, p.bias, (int)n);
-        else
-          p.partial[((int64_t)blockIdx.z * p.M + m) * p.N + n] = v;
+        p.y[(int64_t)m * p.N + n] = finish_output<DT>(v, p.bias, (int)n);
       }
     }
 }
