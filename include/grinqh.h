@@ -202,8 +202,11 @@ int grinqh_time_next_product(void* event_before, void* event_after);
 /* Kernel selection query; no counterpart in the reference (for tests and
  * benchmarks).  Names the kernel that serves an M-row product of this shape
  * through grinqh_gemm_or_gemv (noalloc = 0) or grinqh_gemm_or_gemv_noalloc
- * (noalloc = 1), nothing launched: GRINQH_KERNEL_GEMV (1-4 rows per launch),
- * GRINQH_KERNEL_DECODE (5-64), GRINQH_KERNEL_TALL (the large-batch prefill;
+ * (noalloc = 1), nothing launched: GRINQH_KERNEL_GEMV (1-4 rows),
+ * GRINQH_KERNEL_DECODE (5-64; for both *rows_per_block receives the rows of one
+ * launch, fewer than M where the fixed scratch makes the entry point run row
+ * chunks, and *splits the K ranges of such a launch with 16-byte aligned
+ * planes), GRINQH_KERNEL_TALL (the large-batch prefill;
  * *rows_per_block and *splits receive its plan), GRINQH_KERNEL_LIBRARY (the
  * dense weight and the library GEMM, where the dispatch prefers it; the
  * library's algorithm query at run time can still send the call to the fused

@@ -142,6 +142,27 @@ def test_product_kernel_query(lib, monkeypatch):
         f(512, 4016, 4096)  # K % 32 != 0
 
 
+def test_row_chunks_fit_the_scratch(lib):
+    """Without a workspace the rows of a decode batch run in launches whose
+    counters, partial sums and batch statistic fit the fixed scratch, the last,
+    shorter launch among them: 33 rows of this weight run as 17 and 16, and
+    dense batches of 16 rows are planned with twice the K ranges of 17."""
+    from grinqh import _lib
+    scratch, counters = 64 << 20, 16384
+    for K, N, bits in ((32768, 57344, 8), (53248, 16384, 8), (57344, 57344, 4), (65536, 131072 - 16, 2)):
+        for mode in (_lib.MODE_DENSE, _lib.MODE_UNION):
+            f = lambda M: _lib.product_kernel(M, K, K, N, _lib.DTYPE_F16, bits, 128, mode, True)
+            for M in range(1, 65):
+                rows = f(M)[1]
+                assert 1 <= rows <= M
+                extra = 4 * K if rows < M and mode == _lib.MODE_UNION else 0
+                for m in {rows, M % rows or rows}:
+                    _, whole, splits = f(m)
+                    assert whole == m, (K, N, M, m)
+                    partial = splits * m * N * 4 if splits > 1 else 0
+                    assert counters + partial + extra <= scratch, (K, N, bits, mode, M, m, splits)
+
+
 def test_invalid_arguments_rejected_on_host(lib):
     from grinqh import _lib
     t = _lib.thresholds_f32([0.0] * 4)

@@ -161,6 +161,31 @@ WorkspaceLayout layout_for(int64_t M, int64_t K, int64_t N, int mode, bool allow
   return w;
 }
 
+// Rows per launch of a decode batch in the allocation-free entry point's fixed
+// scratch (a large K forces many K ranges, and the partial sums grow with the
+// rows): halved until the launches fit.  The last launch may have fewer rows
+// than the others and still need more (a smaller batch may be planned with more
+// K ranges), so the layout is the larger of the two.  With one row every valid
+// shape fits.
+struct RowChunks {
+  int64_t rows;
+  WorkspaceLayout layout;
+  size_t bytes;  // the layout, and `extra` bytes after it
+};
+RowChunks plan_row_chunks(int64_t M, int64_t K, int64_t N, int mode, int64_t ldx, int gs, size_t budget,
+                          size_t extra) {
+  RowChunks c{};
+  for (c.rows = M;; c.rows = (c.rows + 1) / 2) {
+    c.layout = layout_for(c.rows, K, N, mode, false, ldx, gs, budget);
+    if (M % c.rows != 0) {
+      const WorkspaceLayout last = layout_for(M % c.rows, K, N, mode, false, ldx, gs, budget);
+      if (last.total > c.layout.total) c.layout = last;
+    }
+    c.bytes = round_up(c.layout.total > kCounterBytes ? c.layout.total : kCounterBytes, 256) + extra;
+    if (c.bytes <= budget || c.rows == 1) return c;
+  }
+}
+
 int check_product_args(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int dtype,
                        const void* planes, const void* scale, void* y, int max_bits, int group_size) {
   if (!valid_dtype(dtype) || !valid_bits(max_bits)) return GRINQH_ERR_INVALID;
@@ -326,26 +351,18 @@ int run_product(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int
   const int mode_l = graded ? GRINQH_MODE_UNION : GRINQH_MODE_DENSE;
   WorkspaceLayout wl = layout_for(M, K, N, mode_l, allow_library, ldx, group_size, allow_library ? 0 : ws_bytes);
   // The allocation-free entry point's fixed scratch may not hold a decode
-  // launch's split-K partial sums (a large K forces many K ranges, and the
-  // partial sums grow with the rows): then the rows run in chunks (halving
-  // until one chunk's layout fits), graded on the statistic of the whole
-  // batch, reduced once into the scratch past the chunks' layout.  With one
-  // row every valid shape fits.
+  // launch's split-K partial sums: then the rows run in chunks (plan_row_chunks),
+  // graded on the statistic of the whole batch, reduced once into the scratch
+  // past the chunks' layout.
   int64_t rows_per_launch = kDecodeMaxRows;
   size_t sigma_off = 0;
   if (!allow_library && M <= kDecodeMaxRows && wl.total > ws_bytes) {
     const size_t sig_bytes = graded && sigma_given == nullptr ? round_up((size_t)K * sizeof(float), 256) : 0;
-    auto need = [&](const WorkspaceLayout& w) {
-      return round_up(w.total > kCounterBytes ? w.total : kCounterBytes, 256) + sig_bytes;
-    };
-    int64_t mc = M;
-    while (mc > 1 && need(wl) > ws_bytes) {
-      mc = (mc + 1) / 2;
-      wl = layout_for(mc, K, N, mode_l, false, ldx, group_size, ws_bytes);
-    }
-    if (need(wl) > ws_bytes) return GRINQH_ERR_SCRATCH;
-    rows_per_launch = mc;
-    sigma_off = need(wl) - sig_bytes;
+    const RowChunks chunks = plan_row_chunks(M, K, N, mode_l, ldx, group_size, ws_bytes, sig_bytes);
+    if (chunks.bytes > ws_bytes) return GRINQH_ERR_SCRATCH;
+    wl = chunks.layout;
+    rows_per_launch = chunks.rows;
+    sigma_off = chunks.bytes - sig_bytes;
   }
   if (wl.total > 0 && (workspace == nullptr || ws_bytes < wl.total || !aligned(workspace, 256)))
     return allow_library ? GRINQH_ERR_WORKSPACE : GRINQH_ERR_SCRATCH;
@@ -615,7 +632,18 @@ int grinqh_product_kernel(int64_t M, int64_t K, int64_t ldx, int64_t N, int dtyp
     return -GRINQH_ERR_INVALID;
   if (rows_per_block != nullptr) *rows_per_block = 0;
   if (splits != nullptr) *splits = 0;
-  if (M <= kDecodeMaxRows) return M <= kGemvMaxRows ? GRINQH_KERNEL_GEMV : GRINQH_KERNEL_DECODE;
+  if (M <= kDecodeMaxRows) {
+    const bool graded = mode == GRINQH_MODE_UNION || (mode == GRINQH_MODE_REFERENCE && M == 1);
+    const int mode_l = graded ? GRINQH_MODE_UNION : GRINQH_MODE_DENSE;
+    int64_t rows = M;
+    if (noalloc != 0 && layout_for(M, K, N, mode_l, false, ldx, group_size, kScratchBytes).total > kScratchBytes)
+      rows = plan_row_chunks(M, K, N, mode_l, ldx, group_size, kScratchBytes,
+                             graded ? round_up((size_t)K * sizeof(float), 256) : 0)
+                 .rows;
+    if (rows_per_block != nullptr) *rows_per_block = (int)rows;
+    if (splits != nullptr) *splits = plan_launch(rows, K, N, group_size, max_bits, !graded, N % 64 == 0).splits;
+    return M <= kGemvMaxRows ? GRINQH_KERNEL_GEMV : GRINQH_KERNEL_DECODE;
+  }
   const bool graded = mode == GRINQH_MODE_UNION;
   const bool allow_library = noalloc == 0;
   const WorkspaceLayout wl = layout_for(M, K, N, graded ? GRINQH_MODE_UNION : GRINQH_MODE_DENSE, allow_library, ldx,
