@@ -348,13 +348,18 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
       const_cast<uint16_t*>(p.x), (short)0, (int)((uint64_t)p.M * p.ldx * 2u), 0x00020000);
   const __amdgpu_buffer_rsrc_t xsrc_none =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.x), (short)0, 0, 0x00020000);
-  // this lane's row, zone and byte offset in a tile for each of the wave's loads
+  // this lane's row, zone and byte offset in a tile for each of the wave's
+  // loads (where the loads do not divide evenly, the last waves' shares end
+  // early: the loads they do not issue repeat the tile's last piece here, so
+  // that every row below is one of the tile's 32)
+  constexpr int G = WB / GB;  // pieces per (e, z, q)
+  constexpr int LAST = IPT * 64 - 1;
+  static_assert(8 * 3 + LAST / (4 * G) / Z < 32, "rows of a tile");
   uint32_t loff[IPW];
   int lrow[IPW], lzone[IPW];
 #pragma unroll
   for (int i = 0; i < IPW; ++i) {
-    constexpr int G = WB / GB;  // pieces per (e, z, q)
-    const int L = (sw * IPW + i) * 64 + lane;
+    const int L = min((sw * IPW + i) * 64 + lane, LAST);
     const int pair = L / (4 * G), rem = L % (4 * G), qq = rem / G;
     const int word = ((rem % G) * GB) ^ (CG == 2 ? 16 * (qq & 1) : 0);
     lrow[i] = 8 * qq + pair / Z;
