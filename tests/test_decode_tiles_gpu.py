@@ -64,3 +64,32 @@ def test_wide_column_blocks(M, gs, mode):
     partial last one (N / 16 = 1804 word columns), and more scale groups than a
     thread keeps in flight."""
     _check(M, 2048, 28864, 8, gs, "float16", mode)
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("mode", ["union", "dense"])
+@pytest.mark.parametrize("M,K,N", [(5, 32, 64), (16, 1024, 1024), (32, 2048, 28864), (33, 160, 400), (64, 2048, 1024)])
+def test_expired_wait_gives_nan(M, K, N, mode, dtype):
+    """A wave that stops waiting for another's share of a tile (here: at once)
+    turns its block's outputs into NaN, and the next call is whole again."""
+    from grinqh import _lib
+    from grinqh.kernel import run_product
+    from grinqh.utils import prepare_weight
+    lib = _lib.load_library()
+    rng = np.random.default_rng(M + K + N)
+    P = prepare_weight(torch.from_numpy(rand_weight(rng, K, N, 8)).cuda(), 8)
+    dt = TORCH_DTYPES[dtype]
+    s = torch.full((-(-K // 32), N), 0.01, dtype=dt, device="cuda")
+    x = torch.from_numpy(rng.standard_normal((M, K))).to(dt).cuda()
+    call = lambda: run_product(x, P, s, None, 8, 32, N // 4, [0.0, 1.2, 1.9, 2.4], mode)
+    want = call()
+    before = lib.grinqh_set_tile_polls(0)
+    try:
+        got = call()
+    finally:
+        assert lib.grinqh_set_tile_polls(before) == 0
+    after = call()
+    torch.cuda.synchronize()
+    assert bool(want.isfinite().all())
+    assert bool(got.isnan().all())
+    assert torch.equal(after, want)

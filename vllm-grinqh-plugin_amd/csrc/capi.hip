@@ -35,6 +35,9 @@ struct KernelEvents {
 };
 KernelEvents g_events;
 
+// Tile handshake polls of this thread's decode launches (grinqh_set_tile_polls).
+thread_local int t_tile_polls = kTilePolls;
+
 }  // namespace
 
 namespace grinqh {
@@ -381,6 +384,7 @@ int run_product(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int
   for (int i = 0; i < 4; ++i) p.thr.t[i] = graded ? thresholds[i] : 0.f;
   p.partial = ws ? reinterpret_cast<float*>(ws + wl.partial_off) : nullptr;
   p.sigma = nullptr;
+  p.tile_polls = t_tile_polls;
 
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   uint16_t* ys = static_cast<uint16_t*>(y);
@@ -665,6 +669,12 @@ int grinqh_time_next_product(void* event_before, void* event_after) {
   g_events.before = static_cast<hipEvent_t>(event_before);
   g_events.after = static_cast<hipEvent_t>(event_after);
   return GRINQH_OK;
+}
+
+int grinqh_set_tile_polls(int polls) {
+  const int before = t_tile_polls;
+  t_tile_polls = polls < 0 || polls > kTilePolls ? kTilePolls : polls;
+  return before;
 }
 
 }  // extern "C"

@@ -127,6 +127,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   __shared__ __align__(16) uint16_t s_scale[SC_GROUPS * 16 * WB];  // (group, tile, column) scales
   __shared__ uint32_t s_smax;  // graded scaled path: largest |scale| (fp16 bits) above the overflow limit
   __shared__ int s_flag[NWV];  // the last tile whose share wave w has in LDS
+  __shared__ int s_late;       // a wave gave up waiting for a share
   // graded, no statistic given: max |x[m][k]| per slice of the batch rows (an
   // entry that is NaN in every row gives 0; every output of such a batch is NaN)
   float* s_sig = reinterpret_cast<float*>(s_pl0);
@@ -136,6 +137,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   const int jg = wave % JG, cg = (wave / JG) % CG, kw = wave / SG;
   const int sw = wave % SG;  // this wave among those of its K sub-range
   if (lane == 0) s_flag[wave] = -(1 << 30);  // read by the others only after the next barrier
+  if (tid == 0) s_late = 0;                  // written by others only after the next barrier
   const int c = lane & 15, q = lane >> 4;
   // logical block = (column block, K range), column blocks fastest, ranges of
   // consecutive logical blocks per XCD (adjacent column blocks share lines)
@@ -426,8 +428,9 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
     // publish it, and wait until every other wave of the K sub-range has
     // published its share, which also means it has read the slots of earlier
     // tiles, the one the next loads overwrite among them.  Every wave
-    // publishes before it waits, so every wait ends (and is bounded: one that
-    // outlasted ~2^22 polls would end, with a wrong tile, rather than hang).
+    // publishes before it waits, so every wait ends.  It is bounded all the
+    // same: a wave that has used up its polls goes on with whatever the slot
+    // holds, all in bounds, and the whole block's outputs become NaN.
     const Zones zn = read_zones(t + PF);
     constexpr int LATER = (PF - 1) * ((IPT % SG == 0 ? IPW : 0) + (MT % SG == 0 ? XPW : 0));
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory");
@@ -435,11 +438,11 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
 #pragma unroll
     for (int pj = 0; pj < SG; ++pj) {
       if (pj == sw) continue;
-      for (int spin = 0; spin < (1 << 22) &&
-                         __builtin_amdgcn_readfirstlane(__hip_atomic_load(
-                             &s_flag[kw * SG + pj], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < t;
-           ++spin) {
-      }
+      int polls = p.tile_polls;
+      while (polls > 0 && __builtin_amdgcn_readfirstlane(__hip_atomic_load(
+                              &s_flag[kw * SG + pj], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < t)
+        --polls;
+      if (polls <= 0) __hip_atomic_store(&s_late, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     asm volatile("" ::: "memory");
     load_tile(t + PF, pnext, xnext, zn);
@@ -551,7 +554,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
     if constexpr (PF == 2) {
       load_tile(t_begin + 1, s_pl1, s_xr1, read_zones(t_begin + 1));
       stage_scales();
-if constexpr (MT == 1) {
+      if constexpr (MT == 1) {
         for (; t + 3 <= t_end; t += 3) {
           step(t, s_pl0, s_xr0, s_pl2, s_xr2);
           step(t + 1, s_pl1, s_xr1, s_pl0, s_xr0);
@@ -633,6 +636,22 @@ if constexpr (MT == 1) {
           }
       }
     }
+  }
+
+  // a wave gave up waiting: a tile may have been multiplied before it was
+  // complete.  One OR per sum leaves it or makes it NaN (a branch or selects
+  // here made the dense 33-64-row kernels spill)
+  static_assert(KW > 1, "the reduction's barriers precede this read");
+  const uint32_t late = s_late != 0 ? 0x7fc00000u : 0u;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    if (!owns(mt)) continue;
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj)
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) Y[mt][jj][b][e] = __uint_as_float(__float_as_uint(Y[mt][jj][b][e]) | late);
   }
 
   // the scaled path multiplies w_eff * s directly: graded rows with a
