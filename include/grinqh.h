@@ -98,7 +98,8 @@ int grinqh_grade(const void* x, int64_t M, int64_t K, int64_t ldx, int dtype, in
  * kernel's regions (a shape the library has no algorithm for runs the
  * hand-written prefill kernels from the same workspace).  It must be zero-filled once before its
  * first use (every call leaves its counters zero again; the rest needs no
- * initial contents), 256-byte aligned, and calls that share it must be
+ * initial contents; the size does not decrease with M up to 64 rows, so a
+ * workspace for one decode batch holds any smaller one), 256-byte aligned, and calls that share it must be
  * ordered (same stream). */
 size_t grinqh_workspace_bytes(int64_t M, int64_t K, int64_t N, int max_bits, int mode);
 

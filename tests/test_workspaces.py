@@ -55,3 +55,23 @@ def test_growth_during_capture_is_refused():
         assert "before graph capture" in str(e)
     else:
         raise AssertionError("growing the workspace under capture must raise")
+
+
+def test_sizes_do_not_decrease_with_the_rows():
+    """A program that has run its largest batch needs no larger workspace for a
+    smaller one, which it could not get under graph capture: dense batches of
+    up to 32 rows are planned with more K ranges than those above."""
+    import random
+    from grinqh import _lib
+    from grinqh.kernel import _workspace_bytes
+    lib = _lib.load_library()
+    rng = random.Random(7)
+    shapes = [(4096, 6144), (4096, 28672), (14336, 4096), (8192, 57344), (28672, 8192), (53248, 16384), (2048, 28864),
+              (32768, 57344), (31104, 20432)]
+    shapes += [(32 * int(2 ** rng.uniform(0, 11)), 16 * int(2 ** rng.uniform(0, 13))) for _ in range(150)]
+    for K, N in shapes:
+        for mode in (_lib.MODE_DENSE, _lib.MODE_UNION, _lib.MODE_REFERENCE):
+            sizes = [lib.grinqh_workspace_bytes(M, K, N, 8, mode) for M in range(65)]
+            assert sizes == sorted(sizes), (K, N, mode)
+            for M in (65, 100, 129, 200, 256, 300, 512):
+                assert _workspace_bytes(lib, M, K, N, 8, mode) >= sizes[64], (K, N, mode, M)

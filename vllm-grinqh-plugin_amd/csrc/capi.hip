@@ -92,6 +92,38 @@ int launch_main(const DecodeParams& p, const DecodePlan& plan, int max_bits, int
                              : launch_decode(p, plan, max_bits, dtype, dense, st);
 }
 
+// Partial-sum bytes of one launch of 1-64 rows, whatever the bit width, the
+// group size and the planes' alignment: only dense batches have a second form
+// (wide column blocks, which 8 bits take wherever fewer bits do).
+size_t launch_partial_bytes(int64_t rows, int64_t K, int64_t N, bool dense) {
+  size_t most = 0;
+  for (const bool wide : {false, true}) {
+    const DecodePlan plan = plan_launch(rows, K, N, 32, 8, dense, wide);
+    if (plan.splits > 1 && plan.workspace > most) most = plan.workspace;
+    if (!dense || rows <= kGemvMaxRows) break;
+  }
+  return most;
+}
+
+// The same for a caller's workspace, non-decreasing in the rows: a smaller batch
+// may be planned with more K ranges, and a caller that has run its largest batch
+// must not need more (under graph capture it could not get it).  Within the row
+// counts that share a plan's form the bytes grow with the rows, except where
+// the cap on partial sums (kMaxPartialBytes) comes near.
+size_t decode_partial_bytes(int64_t M, int64_t K, int64_t N, bool dense) {
+  size_t most = 0;
+  auto add = [&](int64_t rows) {
+    const size_t b = launch_partial_bytes(rows, K, N, dense);
+    most = b > most ? b : most;
+  };
+  for (const int64_t rows : {1, 4, 16, 32})
+    if (rows < M) add(rows);
+  add(M);
+  if (most >= kMaxPartialBytes / 4)
+    for (int64_t rows = 1; rows < M; ++rows) add(rows);
+  return most;
+}
+
 // [split-K counters (kCounterBytes, zero between calls) | sigma (K floats,
 // graded batches above kDecodeMaxRows) | split-K partials | repacked x of
 // the large-batch kernel, or the library-GEMM regions].  The counters sit at
@@ -124,11 +156,7 @@ WorkspaceLayout layout_for(int64_t M, int64_t K, int64_t N, int mode, bool allow
                          (tall_fits ? lib_f16 && lib_bf16 && prefill_prefers_library(M, K, N) : lib_f16 || lib_bf16);
   bool tall_shape = false;
   if (M <= kDecodeMaxRows) {
-    for (const int bits : {2, 8})  // any bit width's plan fits, whatever the planes' alignment
-      for (const bool wide : {false, true}) {
-        const DecodePlan plan = plan_launch(M > 0 ? M : 1, K, N, 32, bits, !g, wide);
-        partial = plan.splits > 1 && plan.workspace > partial ? plan.workspace : partial;
-      }
+    partial = allow_library ? decode_partial_bytes(M, K, N, !g) : launch_partial_bytes(M, K, N, !g);
   } else {  // prefill: partial sums only when its grid is split over K
     tall_shape = !lib_first && tall_fits;
     xt = tall_shape ? round_up(tall_x_bytes(M, K), 256) : 0;

@@ -118,6 +118,16 @@ def _dtype_code(dtype: torch.dtype) -> int:
     raise ValueError(f"GRINQH supports float16 and bfloat16 activations, got {dtype}")
 
 
+def _workspace_bytes(lib, M: int, K: int, N: int, max_bits: int, mode_code: int) -> int:
+    """Workspace of this product and of every smaller decode batch (64 rows and
+    fewer; the library's sizes do not decrease up to there), so that a program
+    which ran its largest batch can capture the others."""
+    nbytes = lib.grinqh_workspace_bytes(M, K, N, max_bits, mode_code)
+    if M > 64:
+        nbytes = max(nbytes, lib.grinqh_workspace_bytes(64, K, N, max_bits, mode_code))
+    return nbytes
+
+
 def run_product(x: torch.Tensor, weight_packed: torch.Tensor, weight_scale: torch.Tensor,
                 bias: Optional[torch.Tensor], max_bits: int, group_size: int, original_n: int,
                 thresholds: List[float], mode: str) -> torch.Tensor:
@@ -153,7 +163,7 @@ def run_product(x: torch.Tensor, weight_packed: torch.Tensor, weight_scale: torc
     lib = _lib.load_library()
     mode_code = _MODES[mode]
     stream = torch._C._cuda_getCurrentRawStream(x.device.index)  # current_stream() without its wrapper object
-    nbytes = lib.grinqh_workspace_bytes(M, K, N, max_bits, mode_code)
+    nbytes = _workspace_bytes(lib, M, K, N, max_bits, mode_code)
     ws = _WORKSPACES.get(x.device, stream, nbytes)
     _lib.check(lib.grinqh_gemm_or_gemv(
         x2.data_ptr(), M, K, x2.stride(0), N, dt, wp.data_ptr(), scale.data_ptr(), bp, y.data_ptr(),
