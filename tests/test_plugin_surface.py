@@ -214,3 +214,31 @@ def test_op_registration_layers():
            16, [0.0] * 4)
     with pytest.raises(RuntimeError, match="no autograd formula"):
         z.sum().backward()
+
+
+_SECOND_COPY = """
+import importlib, importlib.util, sys, types
+import torch
+import grinqh.kernel as first
+importlib.reload(first)
+pkg = types.ModuleType("grinqh_copy")
+pkg.__path__ = list(sys.modules["grinqh"].__path__)
+sys.modules["grinqh_copy"] = pkg
+second = importlib.import_module("grinqh_copy.kernel")
+assert second.__file__ == first.__file__ and second is not first
+assert torch._C._dispatch_has_kernel_for_dispatch_key("grinqh::gemm_or_gemv", "CUDA")
+importlib.reload(first)
+print("loaded")
+"""
+
+
+def test_module_loads_a_second_time():
+    """Two copies of the module in one process (two paths that reach it): the
+    later definition of the op replaces the earlier, device kernel included."""
+    import subprocess
+    import sys
+    import grinqh
+    root = os.path.dirname(os.path.dirname(grinqh.__file__))
+    r = subprocess.run([sys.executable, "-c", _SECOND_COPY], capture_output=True, text=True,
+                       env={**os.environ, "PYTHONPATH": root})
+    assert r.returncode == 0 and r.stdout.strip() == "loaded", r.stderr[-2000:]

@@ -205,9 +205,10 @@ def _gemm_or_gemv_device(x, weight_packed, weight_scale, bias, max_bits, group_s
 # wrapper, which compares the storages of every argument and result on each
 # call (the result here is always a new tensor): 3.5 us of a call's 15 us of
 # dispatch.  Autograd, fake tensors and tracing stay the custom op's; host
-# tensors reach it and are refused there.
-_DEVICE_KERNEL = torch.library.Library("grinqh", "FRAGMENT")
-_DEVICE_KERNEL.impl("gemm_or_gemv", _gemm_or_gemv_device, "CUDA")
+# tensors reach it and are refused there.  It goes into the custom op's own
+# library, so that a second definition of the op (this module loaded again)
+# replaces it together with the first.
+grinqh_gemm_or_gemv._lib.impl("gemm_or_gemv", _gemm_or_gemv_device, "CUDA")
 
 
 def grinqh_gemv_batch_union(x: torch.Tensor, weight_packed: torch.Tensor, weight_scale: torch.Tensor,
