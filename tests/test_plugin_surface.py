@@ -242,3 +242,36 @@ def test_module_loads_a_second_time():
     r = subprocess.run([sys.executable, "-c", _SECOND_COPY], capture_output=True, text=True,
                        env={**os.environ, "PYTHONPATH": root})
     assert r.returncode == 0 and r.stdout.strip() == "loaded", r.stderr[-2000:]
+
+
+def test_device_kernel_is_not_traced(monkeypatch):
+    """Where torch.compile leaves a frame to the interpreter it still looks at
+    what that frame calls: the op's device kernel and its callees are not for
+    it to trace."""
+    import grinqh.kernel as gk
+    traced = []
+
+    def product(x, *args):
+        traced.append(torch.compiler.is_dynamo_compiling())
+        return x + 1
+
+    monkeypatch.setattr(gk, "run_product", product)
+
+    class Unsupported:
+        def __enter__(self):
+            torch._dynamo.graph_break()
+
+        def __exit__(self, *exc):
+            return False
+
+    def frame(x):
+        with Unsupported():  # a break inside a context manager: the frame runs uncompiled
+            torch._dynamo.graph_break()
+            return gk._gemm_or_gemv_device(x, None, None, None, 8, 128, 16, [0.0] * 4)
+
+    torch._dynamo.reset()
+    try:
+        y = torch.compile(frame, backend="eager")(torch.zeros(2))
+    finally:
+        torch._dynamo.reset()
+    assert torch.equal(y, torch.ones(2)) and traced == [False]

@@ -195,6 +195,20 @@ def _fake(x, weight_packed, weight_scale, bias, max_bits, group_size, original_n
     return torch.empty(x.shape[:-1] + (original_n * 4,), device=x.device, dtype=x.dtype)
 
 
+def _untraced(fn):
+    """fn and what it calls, kept from torch.compile's frame evaluator: it
+    reaches a kernel that the dispatcher calls from a frame it could not
+    capture.  Set once on the code object; torch.compiler.disable, which the
+    custom op's wrapper goes through, costs 1 us a call."""
+    try:
+        from torch._C._dynamo.eval_frame import _FrameAction, _FrameExecStrategy, set_code_exec_strategy
+    except ImportError:
+        return torch.compiler.disable(fn)
+    set_code_exec_strategy(fn.__code__, _FrameExecStrategy(_FrameAction.SKIP, _FrameAction.SKIP))
+    return fn
+
+
+@_untraced
 def _gemm_or_gemv_device(x, weight_packed, weight_scale, bias, max_bits, group_size, original_n, thresholds,
                          use_marlin=False):
     return run_product(x, weight_packed, weight_scale, bias, max_bits, group_size, original_n, thresholds,
