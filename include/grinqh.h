@@ -200,15 +200,14 @@ int grinqh_gemm_or_gemv_noalloc(const void* x, int64_t M, int64_t K, int64_t ldx
  * NULLs disarms.  Not for use under graph capture. */
 int grinqh_time_next_product(void* event_before, void* event_after);
 
-/* Error-path instrumentation; no counterpart in the reference.  In products of
- * 5-64 rows the waves of a block wait for each other's share of a tile, each
- * wait bounded by a number of polls (tens of milliseconds; the others' shares
- * take microseconds).  A wait that reaches the bound turns the block's outputs
- * into NaN.  This sets the bound for the calling thread's later launches, so
- * that a test can take that path without a fault (0: every wait counts as
- * having reached it); a negative or larger value restores the default.
- * Returns the bound it replaces. */
-int grinqh_set_tile_polls(int polls);
+/* Error-path instrumentation; no counterpart in the reference.  In most
+ * products of 5-64 rows the waves of a block wait for each other's share of a
+ * tile.  Each wait is bounded (tens of milliseconds; the others' shares take
+ * microseconds), and one that expires turns the block's outputs into NaN.  With
+ * on != 0 the calling thread's later launches treat their waits as expired, so
+ * that a test can take that path; 0 restores the default.  Returns the setting
+ * it replaces. */
+int grinqh_expire_tile_waits(int on);
 
 /* Kernel selection query; no counterpart in the reference (for tests and
  * benchmarks).  Names the kernel that serves an M-row product of this shape

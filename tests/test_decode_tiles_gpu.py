@@ -67,11 +67,13 @@ def test_wide_column_blocks(M, gs, mode):
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
-@pytest.mark.parametrize("mode", ["union", "dense"])
-@pytest.mark.parametrize("M,K,N", [(5, 32, 64), (16, 1024, 1024), (32, 2048, 28864), (33, 160, 400), (64, 2048, 1024)])
+@pytest.mark.parametrize("M,K,N,mode", [
+    (5, 32, 64, "dense"), (16, 1024, 1024, "dense"), (9, 2048, 28864, "union"), (32, 2048, 28864, "dense"),
+    (32, 2048, 28864, "union"), (33, 160, 400, "dense"), (33, 160, 400, "union"), (64, 2048, 1024, "union")])
 def test_expired_wait_gives_nan(M, K, N, mode, dtype):
-    """A wave that stops waiting for another's share of a tile (here: at once)
-    turns its block's outputs into NaN, and the next call is whole again."""
+    """(Forms that share tiles.)  A wait for another wave's share of a tile that
+    expires (here: is taken to) turns its block's outputs into NaN, and the next
+    call is whole again."""
     from grinqh import _lib
     from grinqh.kernel import run_product
     from grinqh.utils import prepare_weight
@@ -83,11 +85,11 @@ def test_expired_wait_gives_nan(M, K, N, mode, dtype):
     x = torch.from_numpy(rng.standard_normal((M, K))).to(dt).cuda()
     call = lambda: run_product(x, P, s, None, 8, 32, N // 4, [0.0, 1.2, 1.9, 2.4], mode)
     want = call()
-    before = lib.grinqh_set_tile_polls(0)
+    assert lib.grinqh_expire_tile_waits(1) == 0
     try:
         got = call()
     finally:
-        assert lib.grinqh_set_tile_polls(before) == 0
+        assert lib.grinqh_expire_tile_waits(0) == 1
     after = call()
     torch.cuda.synchronize()
     assert bool(want.isfinite().all())

@@ -35,8 +35,9 @@ struct KernelEvents {
 };
 KernelEvents g_events;
 
-// Tile handshake polls of this thread's decode launches (grinqh_set_tile_polls).
-thread_local int t_tile_polls = kTilePolls;
+// Whether this thread's decode launches treat their tile waits as expired
+// (grinqh_expire_tile_waits).
+thread_local int t_expire_waits = 0;
 
 }  // namespace
 
@@ -412,7 +413,7 @@ int run_product(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int
   for (int i = 0; i < 4; ++i) p.thr.t[i] = graded ? thresholds[i] : 0.f;
   p.partial = ws ? reinterpret_cast<float*>(ws + wl.partial_off) : nullptr;
   p.sigma = nullptr;
-  p.tile_polls = t_tile_polls;
+  p.expired = t_expire_waits;
 
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   uint16_t* ys = static_cast<uint16_t*>(y);
@@ -699,9 +700,9 @@ int grinqh_time_next_product(void* event_before, void* event_after) {
   return GRINQH_OK;
 }
 
-int grinqh_set_tile_polls(int polls) {
-  const int before = t_tile_polls;
-  t_tile_polls = polls < 0 || polls > kTilePolls ? kTilePolls : polls;
+int grinqh_expire_tile_waits(int on) {
+  const int before = t_expire_waits;
+  t_expire_waits = on != 0 ? 1 : 0;
   return before;
 }
 

@@ -137,7 +137,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   const int jg = wave % JG, cg = (wave / JG) % CG, kw = wave / SG;
   const int sw = wave % SG;  // this wave among those of its K sub-range
   if (lane == 0) s_flag[wave] = -(1 << 30);  // read by the others only after the next barrier
-  if (tid == 0) s_late = 0;                  // written by others only after the next barrier
+  if (tid == 0) s_late = p.expired;          // written by others only after the next barrier
   const int c = lane & 15, q = lane >> 4;
   // logical block = (column block, K range), column blocks fastest, ranges of
   // consecutive logical blocks per XCD (adjacent column blocks share lines)
@@ -417,6 +417,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   int gloc = (tile0 + t_begin) / tiles_per_group - g_first;
   uint32_t s2[NJ][4];  // scaled path: (s, s) of the current group's columns
   const uint16_t dense_value = row_value((1u << Z) - 1u, 0);
+  int polls = 0;  // of all this wave's waits, four at a time
   // one tile: handshake, loads of tile t + PF, unpack, MFMA, group epilogue
   auto step = [&](int t, const unsigned char* pcur, const unsigned char* xcur, unsigned char* pnext, unsigned char* xnext) {
     const bool first_of_group = (t == t_begin) || (gpos == 0);
@@ -429,8 +430,8 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
     // published its share, which also means it has read the slots of earlier
     // tiles, the one the next loads overwrite among them.  Every wave
     // publishes before it waits, so every wait ends.  It is bounded all the
-    // same: a wave that has used up its polls goes on with whatever the slot
-    // holds, all in bounds, and the whole block's outputs become NaN.
+    // same: a wave whose waits have used up their polls goes on with whatever the
+    // slot holds, all in bounds, and the block's outputs become NaN.
     const Zones zn = read_zones(t + PF);
     constexpr int LATER = (PF - 1) * ((IPT % SG == 0 ? IPW : 0) + (MT % SG == 0 ? XPW : 0));
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory");
@@ -438,11 +439,11 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
 #pragma unroll
     for (int pj = 0; pj < SG; ++pj) {
       if (pj == sw) continue;
-      int polls = p.tile_polls;
-      while (polls > 0 && __builtin_amdgcn_readfirstlane(__hip_atomic_load(
-                              &s_flag[kw * SG + pj], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) < t)
-        --polls;
-      if (polls <= 0) __hip_atomic_store(&s_late, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      auto waiting = [&]() {
+        return __builtin_amdgcn_readfirstlane(__hip_atomic_load(&s_flag[kw * SG + pj], __ATOMIC_RELAXED,
+                                                                __HIP_MEMORY_SCOPE_WORKGROUP)) < t;
+      };
+      while (waiting() && waiting() && waiting() && waiting() && polls < kTilePolls) ++polls;
     }
     asm volatile("" ::: "memory");
     load_tile(t + PF, pnext, xnext, zn);
@@ -580,6 +581,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
       }
     }
   }
+  if (polls >= kTilePolls) s_late = 1;  // read after the reduction's barriers
   // the slots are reused below: none of this wave's loads may still be on its
   // way to them (loads past the range leave zeros)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -638,22 +640,6 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
     }
   }
 
-  // a wave gave up waiting: a tile may have been multiplied before it was
-  // complete.  One OR per sum leaves it or makes it NaN (a branch or selects
-  // here made the dense 33-64-row kernels spill)
-  static_assert(KW > 1, "the reduction's barriers precede this read");
-  const uint32_t late = s_late != 0 ? 0x7fc00000u : 0u;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    if (!owns(mt)) continue;
-#pragma unroll
-    for (int jj = 0; jj < NJ; ++jj)
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) Y[mt][jj][b][e] = __uint_as_float(__float_as_uint(Y[mt][jj][b][e]) | late);
-  }
-
   // the scaled path multiplies w_eff * s directly: graded rows with a
   // non-finite activation become NaN, as in the reference
   if constexpr (SC && !DENSE) {
@@ -668,6 +654,26 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
           for (int e = 0; e < 4; ++e) Y[mt][jj][b][e] = graded_nonfinite_to_nan(Y[mt][jj][b][e]);
     }
   }
+
+  // A wave gave up waiting, so a tile may have been multiplied before it was
+  // complete: the block's outputs (or partial sums) are overwritten by NaN.
+  // Apart from the stores of the sums, whose registers a branch around them
+  // would spill.
+  static_assert(KW > 1, "the reduction's barriers precede this read");
+  const bool late = s_late != 0;  // block-uniform
+  auto poison = [&]() {
+    __builtin_amdgcn_s_waitcnt(0);  // the stores of the sums
+#pragma unroll 1
+    for (int i = 0; i < MT * NJ * 16; ++i) {
+      const int mt = i / (NJ * 16), m = 16 * mt + 4 * q + (i & 3);
+      const int64_t n = (int64_t)(4 * jg * NJ + (i / 4) % (4 * NJ)) * p.NW + wc;
+      if (kw != mt % KW || m >= p.M || !col_ok) continue;
+      if (p.splits == 1)
+        p.y[(int64_t)m * p.N + n] = from_f32<DT>(__int_as_float(0x7fc00000));
+      else
+        store_partial(&p.partial[((int64_t)split * p.M + m) * p.N + n], __int_as_float(0x7fc00000));
+    }
+  };
 
   // ---- phase 4: output (direct, or split-K partials + last-block reduction)
   // Output (m, n) of this lane: m = 16*mt + 4*q + e, n = (4*(jg*NJ+jj)+b)*NW + w0 + c.
@@ -689,6 +695,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
             }
       }
     }
+    if (late) poison();
     return;
   }
 
@@ -742,6 +749,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
           }
     }
   }
+  if (late) poison();
   if (p.counters != nullptr) splitk_complete<DT, 1024 * MT * CG / NT, NT>(p, lb % col_blocks, w0, WB);
 }
 

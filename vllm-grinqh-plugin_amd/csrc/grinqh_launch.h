@@ -35,12 +35,13 @@ struct DecodeParams {
   int sigma_chunks;     // arrays at sigma (1 for a plain [K] statistic)
   uint32_t* counters;   // per column block, zero on entry: the kernel completes split-K
                         // itself; nullptr: partial sums only, the reduce kernel follows
-  int tile_polls;       // decode kernel: polls a wave waits for another's share of a tile
+  int expired;          // decode kernel: 1 treats its waits for shares of a tile as expired (tests)
 };
 
-// Polls of the decode kernel's tile handshake: tens of milliseconds, thousands
-// of times the longest wait that other waves of the same block can cause.
-constexpr int kTilePolls = 1 << 22;
+// Polls of the decode kernel's tile handshake that a wave may use (counted in
+// fours): tenths of a second, far beyond all the waits that the other waves of
+// its block can cause.
+constexpr int kTilePolls = 1 << 20;
 
 struct DecodePlan {
   int mt;      // 16-row m-tiles: 1, 2 or 4 (M <= 16, 32, 64)

@@ -57,7 +57,7 @@ SIGNATURES = {
     "grinqh_gemv_batch_union_sigma": (_i32, [_vp, _i64, _i64, _i64, _i64, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _f4,
                                              _vp, _vp, ctypes.c_size_t, _vp]),
     "grinqh_time_next_product": (_i32, [_vp, _vp]),
-    "grinqh_set_tile_polls": (_i32, [_i32]),
+    "grinqh_expire_tile_waits": (_i32, [_i32]),
     "grinqh_product_kernel": (_i32, [_i64, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32,
                                      ctypes.POINTER(_i32), ctypes.POINTER(_i32)]),
 }
