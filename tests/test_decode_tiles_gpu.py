@@ -1,7 +1,8 @@
-"""The decode kernel's tiles in LDS (csrc/decode.hip): its 16- and 32-column
-blocks, 16-byte and 4-byte plane loads, the waves' shares of a tile at every
-bit width, ranges of one to a few tiles, and scale groups past the ones kept in
-flight, against the float64 oracle at the tolerance of the other products."""
+"""The decode kernel's tiles (csrc/decode.hip): its 16- and 32-column blocks,
+plane words through LDS by 16-byte and 4-byte loads and straight into
+registers, the waves' shares of a tile at every bit width, ranges of one to
+many tiles, scale groups past the ones kept in flight and waits that expire,
+against the float64 oracle at the tolerance of the other products."""
 import numpy as np
 import pytest
 import torch
@@ -61,9 +62,95 @@ def test_unaligned_planes(M):
 @pytest.mark.parametrize("M,gs", [(16, 32), (16, 128), (30, 32), (30, 128)])
 def test_wide_column_blocks(M, gs, mode):
     """Weights large enough for 32-column blocks in the dense dispatch, with a
-    partial last one (N / 16 = 1804 word columns), and more scale groups than a
-    thread keeps in flight."""
+    partial last one (N / 16 = 1804 word columns)."""
     _check(M, 2048, 28864, 8, gs, "float16", mode)
+
+
+# ---- large weights: every block runs many tiles, the oracle a part of the columns
+
+_LARGE = {}
+
+
+def _large(K, N, b):
+    """A weight shared by the cases of one shape and width: codes of the
+    checked columns (the first, some in the middle and the last word columns of
+    all 16 column tiles), and the planes of all."""
+    from grinqh.utils import prepare_weight
+    key = (K, N, b)
+    if key not in _LARGE:
+        _LARGE.clear()
+        g = torch.Generator(device="cuda").manual_seed(K + N + b)
+        W = torch.randint(-(1 << (b - 1)), 1 << (b - 1), (K, N), generator=g, device="cuda", dtype=torch.int8)
+        NW = N // 16
+        words = np.r_[0:20, NW // 2:NW // 2 + 20, NW - 20:NW]
+        cols = (np.arange(16)[:, None] * NW + words[None, :]).reshape(-1)
+        ct = torch.from_numpy(cols).cuda()
+        _LARGE[key] = (prepare_weight(W, b), W[:, ct].cpu().numpy(), ct)
+    return _LARGE[key]
+
+
+def _check_large(M, K, N, b, gs, dtype, mode):
+    from grinqh.kernel import run_product
+    P, W, ct = _large(K, N, b)
+    rng = np.random.default_rng(M + b)
+    s = to_dtype_np(np.abs(rng.standard_normal((-(-K // gs), N))) * 0.02 + 1e-3, dtype)
+    x = to_dtype_np(rng.standard_normal((M, K)), dtype)
+    t = [0.0] + np.quantile(np.abs(x).max(0), [0.5, 0.8, 0.95]).tolist()
+    dt = TORCH_DTYPES[dtype]
+    xt, st = torch.from_numpy(x).to(dt).cuda(), torch.from_numpy(s).to(dt).cuda()
+    y = run_product(xt, P, st, None, b, gs, N // 4, t, mode)
+    again = run_product(xt, P, st, None, b, gs, N // 4, t, mode)
+    torch.cuda.synchronize()
+    assert torch.equal(y, again), "not repeatable"
+    cols = ct.cpu().numpy()
+    pre = own_product(x, W, s[:, cols], t, b, gs, dtype, mode == "union")
+    assert_output_close(y[:, ct], pre, to_dtype_np(pre, dtype), dtype, what=f"{M}x{K}x{N} b={b} {mode} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("mode", ["union", "dense"])
+@pytest.mark.parametrize("M", [16, 32, 64])
+@pytest.mark.parametrize("N", [28864, 28848])
+@pytest.mark.parametrize("b", [2, 4, 6, 8])
+def test_slots_are_reused(b, N, M, mode, dtype):
+    """1000 and more rows of K per block, 8 to 16 tiles and more per sub-range:
+    every LDS slot and tile buffer is filled and read several times, at every
+    bit width (uneven shares among four waves at 6 bits in bf16), with 16-byte
+    plane loads (28864 columns; dense 4-8 bits at 16 rows and 6-8 bits at 32:
+    blocks of 32 word columns) and 4-byte or direct ones (28848)."""
+    _check_large(M, 4096, N, b, 128, dtype, mode)
+
+
+@pytest.mark.parametrize("mode", ["union", "dense"])
+@pytest.mark.parametrize("M", [16, 30, 64])
+def test_scale_groups_past_the_ones_in_flight(M, mode):
+    """Groups of 32 rows: 64 per block (graded, and 33-64 rows) where a thread
+    keeps 32 in flight, 32 per block of 32 word columns where it keeps 24."""
+    _check_large(M, 4096, 28864, 8, 32, "float16", mode)
+
+
+@pytest.mark.parametrize("M", [20, 64])
+def test_overflow_guard_sees_late_scale_groups(M):
+    """The one scale past the fp16 weight range lies in group 40 of its block,
+    stored ahead of the first barrier with the groups that are not kept in
+    flight."""
+    from grinqh.kernel import grinqh_gemv_batch_union
+    from oracle import grinqh_oracle as O
+    K, N, b, gs = 4096, 28864, 8, 32
+    P, W, ct = _large(K, N, b)
+    cols = ct.cpu().numpy()
+    rng = np.random.default_rng(M)
+    s = np.full((K // gs, N), 0.25)
+    s[40, cols[::3]] = 1500.0
+    x = to_dtype_np(rng.standard_normal((M, K)) * 1e-3, "float16")
+    t = [0.0] + np.quantile(np.abs(x).max(0), [0.5, 0.8, 0.95]).tolist()
+    y = grinqh_gemv_batch_union(torch.from_numpy(x).half().cuda(), P, torch.from_numpy(s).half().cuda(), None, b, gs,
+                                N // 4, t)
+    weff = O.effective_weight(W, O.grade(O.union_sigma(x), t, b), b).astype(np.float64)
+    m, e = np.frexp(weff * np.repeat(s[:, cols], gs, axis=0))  # 11 significant bits, no exponent limit
+    pre = x @ np.ldexp(np.round(m * 2.0 ** 11) / 2.0 ** 11, e)
+    assert np.abs(pre).max() < 65504
+    assert_output_close(y[:, ct], pre, to_dtype_np(pre, "float16"), "float16", what=f"late scale group M={M}")
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
