@@ -235,3 +235,14 @@ def test_noalloc_rejects_mode_and_thresholds_before_device_state(lib):
     assert call(_lib.MODE_UNION, None) == _lib.GRINQH_ERR_INVALID            # graded: thresholds required
     assert call(_lib.MODE_REFERENCE, None, M=1) == _lib.GRINQH_ERR_INVALID   # one row is graded
     assert call(_lib.MODE_UNION, t, M=0) == _lib.GRINQH_OK                   # empty batch: nothing to do
+
+
+def test_short_k_ranges_fill_the_gpu(lib):
+    """Products of 17-32 rows split a short K into ranges of two tiles for each
+    of two sub-ranges, as far as the compute units go: 1024 x 2560 (10 column
+    blocks) into 8, 2816 x 1024 into 22 and 4096 x 1024 into 32."""
+    from grinqh import _lib
+    for M in (17, 32):
+        for dtype in (_lib.DTYPE_F16, _lib.DTYPE_BF16):
+            for K, N, want in ((1024, 2560, 8), (2816, 1024, 22), (4096, 1024, 32), (4096, 6144, 10)):
+                assert _lib.product_kernel(M, K, K, N, dtype, 8, 128, _lib.MODE_UNION)[2] == want, (M, K, N)
