@@ -117,7 +117,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   constexpr int RED_PER = (RED_SLOTS + RED_ARRAYS - 1) / RED_ARRAYS;
   constexpr int PL_BYTES = KW * TILE > RED_PER * RED_SLOT ? KW * TILE : RED_PER * RED_SLOT;
   constexpr int XR_BYTES = KW * MT * 1024;
-  constexpr int SIG_BYTES = NT * 8 * 4;  // at most NT / U slices of U chunks of 8 rows
+  constexpr int SIG_BYTES = MT > 1 && !DENSE ? NT * 8 * 4 : 0;  // at most NT / U slices of U chunks of 8 rows
   __shared__ __align__(16) unsigned char s_pl0[PL_BYTES > SIG_BYTES ? PL_BYTES : SIG_BYTES];
   __shared__ __align__(16) unsigned char s_pl1[PL_BYTES];
   __shared__ __align__(16) unsigned char s_pl2[PF == 2 ? PL_BYTES : 16];
@@ -130,7 +130,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   __shared__ uint32_t s_smax;  // graded scaled path: largest |scale| (fp16 bits) above the overflow limit
   __shared__ int s_flag[NWV];  // the last tile whose share wave w has in LDS
   __shared__ int s_late;       // a wave gave up waiting for a share
-  // graded, no statistic given: max |x[m][k]| per slice of the batch rows (an
+  // graded, 17-64 rows, no statistic given: max |x[m][k]| per slice of the batch rows (an
   // entry that is NaN in every row gives 0; every output of such a batch is NaN)
   float* s_sig = reinterpret_cast<float*>(s_pl0);
 
@@ -165,7 +165,28 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   uint32_t smax = 0;  // largest |scale| bits this thread staged
   if (GUARD && threadIdx.x == 0) s_smax = 0;
   const bool own_sigma = !DENSE && p.sigma == nullptr;  // block-uniform
-  const int sig_slices = min(NT / (R >> 3), p.M);  // batch rows are dealt to this many threads per K chunk
+  // (more than 16 rows) batch rows are dealt to this many threads per K chunk,
+  // two or more rows each: fewer slices to take the maximum of
+  const int sig_slices = min(NT / (R >> 3), (p.M + 1) >> 1);
+
+  // Grading a row: zone bits, correction-column value and zone-0 flip.  Rows
+  // with zone 0 active are consumed in offset binary (zone 0's digits flipped,
+  // u = int8(U & mask) + 128, and the column value removes the 128); other rows
+  // have bit 7 clear and need no flip:
+  //   w_eff * 2^sh = u + beta * 2^sh - (zone 0 active ? 128 : 0).
+  // A row with no active zone therefore contributes exact zeros.  Dense, every
+  // row has the same constants.
+  auto row_value = [&](uint32_t bits, int beta) -> uint16_t {
+    if constexpr (SC)  // -c_row of the scaled weight (u >> sh) - c_row, an exact fp16 integer
+      return f32_to_f16_bits(-(float)(1024 + ((bits & 1u) ? (128 >> SH) : 0) - beta));
+    else
+      return BOperand<DT>::correction(beta * (1 << SH) - ((bits & 1u) ? 128 : 0));
+  };
+  auto grade_row = [&](int rr, float s) {
+    const uint32_t bits = zone_bits<Z>(s, p.thr.t);
+    s_bv[rr] = row_value(bits, midpoint_bias<Z>(bits));
+    s_zb[rr] = (uint8_t)(bits | ((bits ^ 15u) << 4));
+  };
 
   // ---- phase 1a: reduce the block's statistic from x and load the scales.
   // The scales are stored to LDS only once the first tiles' loads are issued,
@@ -181,11 +202,11 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
     const uint32_t sbytes = (uint32_t)((uint64_t)((p.K + p.gs - 1) / p.gs) * p.N * 2u);
     const __amdgpu_buffer_rsrc_t sr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint16_t*>(p.scale), (short)0, (int)sbytes, 0x00020000);
-    // the block's statistic: thread t takes K chunk u0 = t % U (8 rows of K)
-    // for batch rows t / U, t / U + S, ... (U = R / 8 <= NT chunks, S slices),
-    // 8 loads at a time, and leaves its maxima in LDS; whoever grades a row
-    // takes the maximum over the slices
-    if (own_sigma) {
+    // the block's statistic above 16 rows: thread t takes K chunk u0 = t % U (8
+    // rows of K) for batch rows t / U, t / U + S, ... (U = R / 8 <= NT chunks, S
+    // slices), 8 loads at a time, and leaves its maxima in LDS; whoever grades a
+    // row takes the maximum over the slices
+    if (MT > 1 && own_sigma) {
       const int U = R >> 3, S = sig_slices;
       const int u0 = tid % U, sl = tid / U;
       if (sl < S) {
@@ -215,16 +236,59 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
         dst[1] = f32x4_t{mx[4], mx[5], mx[6], mx[7]};
       }
     }
+    auto load_scales = [&]() {
 #pragma unroll
-    for (int k = 0; k < SPT; ++k) {
-      const int h = tid + NT * k;  // (group, tile, half) chunk
-      const int gl = h / (32 * CG), r = (h / (2 * CG)) & 15, hf = h % (2 * CG);
-      const uint32_t off =
-          (gl < n_groups && vec_scales)
-              ? (uint32_t)(((int64_t)(g_first + gl) * p.N + (int64_t)r * p.NW + w0 + 8 * hf) * 2)
-              : 0x80000000u;
-      sv[k] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, (int)off, 0, 0));
-    }
+      for (int k = 0; k < SPT; ++k) {
+        const int h = tid + NT * k;  // (group, tile, half) chunk
+        const int gl = h / (32 * CG), r = (h / (2 * CG)) & 15, hf = h % (2 * CG);
+        const uint32_t off =
+            (gl < n_groups && vec_scales)
+                ? (uint32_t)(((int64_t)(g_first + gl) * p.N + (int64_t)r * p.NW + w0 + 8 * hf) * 2)
+                : 0x80000000u;
+        sv[k] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(sr, (int)off, 0, 0));
+      }
+    };
+    // Up to 16 rows a thread takes two K rows (four where the K range is longer
+    // than two per thread) of every batch row, all loads in flight, and grades
+    // them from registers: no slices in LDS, one barrier less (batch rows past
+    // the last repeat it; a NaN is ignored as fmaxf does).  16 rows graded:
+    // down 19.3 -> 18.3 us, gate_up 30.2 -> 29.5.
+    auto grade_rows = [&](auto words) {
+      constexpr int W = decltype(words)::value;  // two K rows each
+      const int rr = 2 * W * tid;
+      uint32_t v[16][W];
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        const int row_off = (int)(((int64_t)min(m, p.M - 1) * p.ldx + row0) * 2);
+        const int off = rr < R ? rr * 2 : (int)0x80000000u;
+        if constexpr (W == 1) {
+          v[m][0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(xr, off, row_off, 0);
+        } else {
+          const u32x2_t u = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(xr, off, row_off, 0));
+          v[m][0] = u[0];
+          v[m][1] = u[1];
+        }
+      }
+      load_scales();
+      if (rr >= R) return;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        float lo = 0.f, hi = 0.f;
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+          lo = fmaxf(lo, fabsf(to_f32<DT>((uint16_t)(v[m][w] & 0xFFFFu))));
+          hi = fmaxf(hi, fabsf(to_f32<DT>((uint16_t)(v[m][w] >> 16))));
+        }
+        grade_row(rr + 2 * w, lo);
+        grade_row(rr + 2 * w + 1, hi);
+      }
+    };
+    if (MT > 1 || !own_sigma)
+      load_scales();
+    else if (R <= 2 * NT)
+      grade_rows(std::integral_constant<int, 1>{});
+    else
+      grade_rows(std::integral_constant<int, 2>{});
     // more groups than those (short groups, long K ranges): stored at once
     for (int h = tid + NT * SPT; h < n_groups * 32 * CG && vec_scales; h += NT) {
       const int gl = h / (32 * CG), r = (h / (2 * CG)) & 15, hf = h % (2 * CG);
@@ -239,29 +303,14 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   }
   __syncthreads();
 
-  // ---- phase 1b (graded): grade each row: zone bits, correction-column value
-  // and zone-0 flip.  Rows with zone 0 active are consumed in offset binary
-  // (zone 0's digits flipped, u = int8(U & mask) + 128, and the column value
-  // removes the 128); other rows have bit 7 clear and need no flip:
-  //   w_eff * 2^sh = u + beta * 2^sh - (zone 0 active ? 128 : 0).
-  // A row with no active zone therefore contributes exact zeros.  Dense, every
-  // row has the same constants.
-  auto row_value = [&](uint32_t bits, int beta) -> uint16_t {
-    if constexpr (SC)  // -c_row of the scaled weight (u >> sh) - c_row, an exact fp16 integer
-      return f32_to_f16_bits(-(float)(1024 + ((bits & 1u) ? (128 >> SH) : 0) - beta));
-    else
-      return BOperand<DT>::correction(beta * (1 << SH) - ((bits & 1u) ? 128 : 0));
-  };
+  // ---- phase 1b (graded, unless graded above): grade each row.
   if constexpr (!DENSE) {
     // (the loop that reads the caller's statistic from global memory is kept
     // apart, so that the other has no global load and the scale loads stay in
     // flight through it)
-    auto grade_row = [&](int rr, float s) {
-      const uint32_t bits = zone_bits<Z>(s, p.thr.t);
-      s_bv[rr] = row_value(bits, midpoint_bias<Z>(bits));
-      s_zb[rr] = (uint8_t)(bits | ((bits ^ 15u) << 4));
-    };
-    if (own_sigma) {  // this block's share of the batch statistic
+    if (MT == 1 && own_sigma) {
+      // graded from registers
+    } else if (own_sigma) {  // this block's share of the batch statistic
       for (int rr = tid; rr < R; rr += NT) {
         float sg = 0.f;
         for (int s0 = 0; s0 < sig_slices; s0 += 8) {  // eight reads in flight (past the last slice: that one again)
@@ -276,7 +325,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
     } else {  // the batch statistic given by the caller
       for (int rr = tid; rr < R; rr += NT) grade_row(rr, precomputed_sigma(p, row0 + rr));
     }
-    __syncthreads();
+    if (MT > 1 || !own_sigma) __syncthreads();
   }
 
   int up_exp = 0;  // the block's sums are scaled by 2^up_exp at the end
