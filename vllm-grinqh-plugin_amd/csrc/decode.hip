@@ -79,9 +79,11 @@ constexpr int decode_rows_per_block(int cg) { return cg == 2 ? 1024 : 2048; }
 template <typename DT, int MT>
 constexpr int decode_dword_groups() { return !decode_scaled<DT, MT>() && MT == 4 ? 4 : 2; }
 
-// CG: groups of 16 word columns per block.  WIDE: plane rows 16-byte aligned
-// (16-byte loads of four words), else 4-byte loads
-template <typename DT, int MT, int Z, bool DENSE, bool WIDE, int CG>
+// CG: groups of 16 word columns per block.  GB: words per lane and load into
+// LDS: 4 (plane rows 16-byte aligned) or 1; or 0, up to 16 rows: each wave loads
+// the words of its own tiles into registers, and x is staged whole (plan_decode
+// says where)
+template <typename DT, int MT, int Z, bool DENSE, int GB, int CG>
 __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodeParams p) {
   constexpr bool SC = decode_scaled<DT, MT>();
   constexpr int NWV = kDecodeWaves;
@@ -91,6 +93,8 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   constexpr int NJ = 4 / JG;           // output dwords j per wave
   constexpr int SG = CG * JG;          // waves per K sub-range
   constexpr int KW = NWV / SG;         // K sub-ranges per block
+  constexpr bool DIRECT = GB == 0;
+  static_assert(!DIRECT || (MT == 1 && CG == 1), "x is staged for 16 rows");
   constexpr int SH = 8 - 2 * Z;
   constexpr int RMAX = decode_rows_per_block(CG);
   static_assert(RMAX / 8 <= NT, "one statistic chunk per thread");
@@ -106,17 +110,25 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   // words at one offset plus constants, without bank conflicts (with 32 word
   // columns the two halves are swapped for odd q).
   constexpr int PF = (MT == 4 && SC ? 1 : 2);
-  constexpr int GB = WIDE ? 4 : 1;                   // words per lane and load
+  constexpr int GL = DIRECT ? 1 : GB;                // words per lane and load
   constexpr int TILE = 32 * Z * WB * 4;              // bytes of one sub-range's tile
-  constexpr int IPT = TILE / (64 * GB * 4);          // loads per tile
+  constexpr int IPT = TILE / (64 * GL * 4);          // loads per tile
   constexpr int IPW = (IPT + SG - 1) / SG;           // at most per wave
   constexpr int XPW = (MT + SG - 1) / SG;            // x fragments per wave, at most
   constexpr int RED_SLOT = NJ * 4 * 64 * 16;         // one wave's sums of an m-tile
   constexpr int RED_SLOTS = (KW - 1) * SG;
   constexpr int RED_ARRAYS = PF + 1;
   constexpr int RED_PER = (RED_SLOTS + RED_ARRAYS - 1) / RED_ARRAYS;
-  constexpr int PL_BYTES = KW * TILE > RED_PER * RED_SLOT ? KW * TILE : RED_PER * RED_SLOT;
-  constexpr int XR_BYTES = KW * MT * 1024;
+  constexpr int PL_BYTES = DIRECT ? 16 : KW * TILE > RED_PER * RED_SLOT ? KW * TILE : RED_PER * RED_SLOT;
+  constexpr int XR_BYTES = DIRECT ? 16 : KW * MT * 1024;
+  // DIRECT: x of the whole K range, fragments of 1 KiB per tile (lane l's 16
+  // bytes at byte 16 l), and, graded, each (row, plane)'s byte offset, bit 31 set
+  // where the row does not need it
+  constexpr int ZS = Z == 3 ? 4 : Z;
+  constexpr int XS_BYTES = DIRECT ? RMAX / 32 * 1024 : 16;
+  static_assert(!DIRECT || RED_SLOTS * RED_SLOT <= XS_BYTES, "the reduction reuses the staged x");
+  __shared__ __align__(16) unsigned char s_xs[XS_BYTES];
+  __shared__ __align__(16) uint32_t s_off[DIRECT && !DENSE ? RMAX * ZS : 4];
   constexpr int SIG_BYTES = MT > 1 && !DENSE ? NT * 8 * 4 : 0;  // at most NT / U slices of U chunks of 8 rows
   __shared__ __align__(16) unsigned char s_pl0[PL_BYTES > SIG_BYTES ? PL_BYTES : SIG_BYTES];
   __shared__ __align__(16) unsigned char s_pl1[PL_BYTES];
@@ -139,7 +151,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   const int jg = wave % JG, cg = (wave / JG) % CG, kw = wave / SG;
   const int sw = wave % SG;  // this wave among those of its K sub-range
   if (lane == 0) s_flag[wave] = -(1 << 30);  // read by the others only after the next barrier
-  if (tid == 0) s_late = p.expired;          // written by others only after the next barrier
+  if (tid == 0) s_late = DIRECT ? 0 : p.expired;          // written by others only after the next barrier
   const int c = lane & 15, q = lane >> 4;
   // logical block = (column block, K range), column blocks fastest, ranges of
   // consecutive logical blocks per XCD (adjacent column blocks share lines)
@@ -186,9 +198,16 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
     const uint32_t bits = zone_bits<Z>(s, p.thr.t);
     s_bv[rr] = row_value(bits, midpoint_bias<Z>(bits));
     s_zb[rr] = (uint8_t)(bits | ((bits ^ 15u) << 4));
+    if constexpr (DIRECT) {
+      const uint32_t row_off = (uint32_t)(row0 + rr) * (uint32_t)(Z * p.NW) * 4u;
+#pragma unroll
+      for (int z = 0; z < Z; ++z)
+        s_off[rr * ZS + z] = ((bits >> z) & 1u) ? row_off + (uint32_t)(z * p.NW) * 4u : 0x80000000u;
+    }
   };
 
-  // ---- phase 1a: reduce the block's statistic from x and load the scales.
+  // ---- phase 1a: reduce the block's statistic from x (and stage x for direct
+  // loads) and load the scales.
   // The scales are stored to LDS only once the first tiles' loads are issued,
   // so their memory round trip overlaps those loads; they are loaded after
   // every x load, so that waiting for x does not wait for them.  Out-of-range
@@ -234,6 +253,13 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
         f32x4_t* dst = reinterpret_cast<f32x4_t*>(&s_sig[sl * R + 8 * u0]);
         dst[0] = f32x4_t{mx[0], mx[1], mx[2], mx[3]};
         dst[1] = f32x4_t{mx[4], mx[5], mx[6], mx[7]};
+      }
+    }
+    if constexpr (DIRECT) {
+      for (int t = wave; t < nt; t += NWV) {  // rows past the batch read 0
+        const uint32_t off = c < p.M ? (uint32_t)(((int64_t)c * p.ldx + row0 + t * 32 + 8 * q) * 2) : 0x80000000u;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            xr, (__attribute__((address_space(3))) void*)(s_xs + t * 1024), 16, (int)off, 0, 0, 0);
       }
     }
     auto load_scales = [&]() {
@@ -301,6 +327,9 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
       }
     }
   }
+  // (direct: this wave's part of x has arrived, the scales loaded after it may
+  // still be on their way)
+  if constexpr (DIRECT) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SPT) : "memory");
   __syncthreads();
 
   // ---- phase 1b (graded, unless graded above): grade each row.
@@ -408,7 +437,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   // load before: gate_up at N = 28688, 8 rows graded, 37.7 -> 35.9 us).
   // Uneven (6 bits, four waves), the last waves' shares end early: the loads
   // they do not issue repeat the tile's last piece here.
-  constexpr int G = WB / GB;  // pieces per (e, z, q)
+  constexpr int G = WB / GL;  // pieces per (e, z, q)
   constexpr bool EVEN = IPT % SG == 0;
   constexpr int RW = EVEN ? 8 / SG : 8;
   constexpr int LAST = IPT * 64 - 1;
@@ -421,9 +450,9 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
 #pragma unroll
   for (int i = 0; i < IPW; ++i) {
     const int pair = EVEN ? i * (64 / (4 * G)) + lane / (4 * G) : min((sw * IPW + i) * 64 + lane, LAST) / (4 * G);
-    const int word = ((lane % G) * GB) ^ (CG == 2 ? 16 * (lq & 1) : 0);
+    const int word = ((lane % G) * GL) ^ (CG == 2 ? 16 * (lq & 1) : 0);
     const int row = 8 * lq + e0 + pair / Z, z = pair % Z;
-    loff[i] = (uint32_t)row * row_bytes + (uint32_t)(z * p.NW + min(w0 + word, p.NW - GB)) * 4u;
+    loff[i] = (uint32_t)row * row_bytes + (uint32_t)(z * p.NW + min(w0 + word, p.NW - GL)) * 4u;
     lbit[i] = 8 * (pair / Z) + 4 + z;
   }
   typedef __attribute__((address_space(3))) void* lds_t;
@@ -454,11 +483,38 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
       if (IPT % SG != 0 && gi >= IPT) break;  // wave-uniform
       uint32_t off = loff[i];
       if constexpr (!DENSE) off |= (uint32_t)(zn >> lbit[i]) << 31;
-      const lds_t dst = (lds_t)(pl + kw * TILE + gi * 64 * GB * 4);
-      if constexpr (WIDE)
+      const lds_t dst = (lds_t)(pl + kw * TILE + gi * 64 * GL * 4);
+      if constexpr (GB == 4)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 16, (int)off, sbase, 0, 0);
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, (int)off, sbase, 0, 0);
+    }
+  };
+  // DIRECT: the words of tile t that this lane multiplies (zeros past the range
+  // and where the grading needs none)
+  struct Tile {
+    uint32_t D[8][Z];
+  };
+  auto load_words = [&](int t, Tile& T) {
+    const bool live = t < t_end;
+    const int tt = live ? t : t_begin;
+    const __amdgpu_buffer_rsrc_t rs = live ? prsrc : prsrc_none;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      typedef uint32_t offs_t __attribute__((ext_vector_type(ZS)));
+      offs_t o = {};
+      if constexpr (!DENSE) o = *reinterpret_cast<const offs_t*>(&s_off[(tt * 32 + 8 * q + e) * ZS]);
+#pragma unroll
+      for (int z = 0; z < Z; ++z) {
+        uint32_t off = (uint32_t)wc * 4u, base = 0;
+        if constexpr (DENSE) {
+          off += (uint32_t)(8 * q) * row_bytes;
+          base = (uint32_t)(row0 + tt * 32 + e) * row_bytes + (uint32_t)(z * p.NW) * 4u;  // wave-uniform
+        } else {
+          off += o[z];
+        }
+        T.D[e][z] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, (int)base, 0);
+      }
     }
   };
   // the LDS words this lane reads of a tile
@@ -471,47 +527,11 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   uint32_t s2[NJ][4];  // scaled path: (s, s) of the current group's columns
   const uint16_t dense_value = row_value((1u << Z) - 1u, 0);
   int polls = 0;  // of all this wave's waits, four at a time
-  // one tile: handshake, loads of tile t + PF, unpack, MFMA, group epilogue
-  auto step = [&](int t, const unsigned char* pcur, const unsigned char* xcur, unsigned char* pnext, unsigned char* xnext) {
+  // one tile from its words and x: unpack, MFMA, group epilogue
+  auto multiply = [&](int t, const u32x4_t (&A)[MT], uint32_t (&D)[8][Z]) __attribute__((always_inline)) {
     const bool first_of_group = (t == t_begin) || (gpos == 0);
     const bool last_of_group = (t + 1 == t_end) || (gpos + 1 == tiles_per_group);
     const int sb = t * 32 + 8 * q;
-
-    // own share of tile t: wait until at most the loads issued after it are in
-    // flight (every wave's share of them, at least).  Then the handshake:
-    // publish it, and wait until every other wave of the K sub-range has
-    // published its share, which also means it has read the slots of earlier
-    // tiles, the one the next loads overwrite among them.  Every wave
-    // publishes before it waits, so every wait ends.  It is bounded all the
-    // same: a wave whose waits have used up their polls goes on with whatever the
-    // slot holds, all in bounds, and the block's outputs become NaN.
-    const zones_t zn = read_zones(t + PF);
-    constexpr int LATER = (PF - 1) * ((IPT % SG == 0 ? IPW : 0) + (MT % SG == 0 ? XPW : 0));
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory");
-    if (lane == 0) __hip_atomic_store(&s_flag[wave], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-#pragma unroll
-    for (int pj = 0; pj < SG; ++pj) {
-      if (pj == sw) continue;
-      auto waiting = [&]() {
-        return __builtin_amdgcn_readfirstlane(__hip_atomic_load(&s_flag[kw * SG + pj], __ATOMIC_RELAXED,
-                                                                __HIP_MEMORY_SCOPE_WORKGROUP)) < t;
-      };
-      while (waiting() && waiting() && waiting() && waiting() && polls < kTilePolls) ++polls;
-    }
-    asm volatile("" ::: "memory");
-    load_tile(t + PF, pnext, xnext, zn);
-    __builtin_amdgcn_sched_barrier(0);
-
-    u32x4_t A[MT];  // x[16*mt + c][rows 8q .. 8q+7 of the tile]
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      A[mt] = *reinterpret_cast<const u32x4_t*>(xcur + (kw * MT + mt) * 1024 + lane * 16);
-    uint32_t D[8][Z];
-#pragma unroll
-    for (int e = 0; e < 8; ++e)
-#pragma unroll
-      for (int z = 0; z < Z; ++z)
-        D[e][z] = *reinterpret_cast<const uint32_t*>(pcur + dpos + (e * Z + z) * 16 * WB);
 
     // Rebuild the code bytes (offset binary) and turn them into B operands.
     u32x4_t bv;
@@ -601,11 +621,72 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
       ++gpos;
     }
   };
+  // one tile through LDS: handshake, loads of tile t + PF, then the tile
+  auto step = [&](int t, const unsigned char* pcur, const unsigned char* xcur, unsigned char* pnext,
+                  unsigned char* xnext) __attribute__((always_inline)) {
+    // own share of tile t: wait until at most the loads issued after it are in
+    // flight (every wave's share of them, at least).  Then the handshake:
+    // publish it, and wait until every other wave of the K sub-range has
+    // published its share, which also means it has read the slots of earlier
+    // tiles, the one the next loads overwrite among them.  Every wave
+    // publishes before it waits, so every wait ends.  It is bounded all the
+    // same: a wave whose waits have used up their polls goes on with whatever the
+    // slot holds, all in bounds, and the block's outputs become NaN.
+    const zones_t zn = read_zones(t + PF);
+    constexpr int LATER = (PF - 1) * ((IPT % SG == 0 ? IPW : 0) + (MT % SG == 0 ? XPW : 0));
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory");
+    if (lane == 0) __hip_atomic_store(&s_flag[wave], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+#pragma unroll
+    for (int pj = 0; pj < SG; ++pj) {
+      if (pj == sw) continue;
+      auto waiting = [&]() {
+        return __builtin_amdgcn_readfirstlane(__hip_atomic_load(&s_flag[kw * SG + pj], __ATOMIC_RELAXED,
+                                                                __HIP_MEMORY_SCOPE_WORKGROUP)) < t;
+      };
+      while (waiting() && waiting() && waiting() && waiting() && polls < kTilePolls) ++polls;
+    }
+    asm volatile("" ::: "memory");
+    load_tile(t + PF, pnext, xnext, zn);
+    __builtin_amdgcn_sched_barrier(0);
+
+    u32x4_t A[MT];  // x[16*mt + c][rows 8q .. 8q+7 of the tile]
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      A[mt] = *reinterpret_cast<const u32x4_t*>(xcur + (kw * MT + mt) * 1024 + lane * 16);
+    uint32_t D[8][Z];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int z = 0; z < Z; ++z)
+        D[e][z] = *reinterpret_cast<const uint32_t*>(pcur + dpos + (e * Z + z) * 16 * WB);
+    multiply(t, A, D);
+  };
 
   {
     int t = t_begin;
-    load_tile(t_begin, s_pl0, s_xr0, read_zones(t_begin));
-    if constexpr (PF == 2) {
+    if constexpr (DIRECT) {
+      // three tile buffers: tiles t + 1 and t + 2 are in flight while tile t is
+      // unpacked
+      auto own_step = [&](int t1, Tile& cur, Tile& next, bool more) __attribute__((always_inline)) {
+        if (more) load_words(t1 + 2, next);
+        __builtin_amdgcn_sched_barrier(0);
+        const u32x4_t A[1] = {*reinterpret_cast<const u32x4_t*>(s_xs + t1 * 1024 + lane * 16)};
+        multiply(t1, A, cur.D);
+      };
+      Tile TA, TB, TC;
+      load_words(t_begin, TA);
+      load_words(t_begin + 1, TB);
+      stage_scales();
+      for (; t + 3 <= t_end; t += 3) {
+        own_step(t, TA, TC, true);
+        own_step(t + 1, TB, TA, true);
+        own_step(t + 2, TC, TB, true);
+      }
+      // at most two tiles left, already loaded into TA and TB
+      if (t < t_end) own_step(t, TA, TC, false);
+      if (t + 1 < t_end) own_step(t + 1, TB, TA, false);
+    } else if constexpr (PF == 2) {
+      load_tile(t_begin, s_pl0, s_xr0, read_zones(t_begin));
       load_tile(t_begin + 1, s_pl1, s_xr1, read_zones(t_begin + 1));
       stage_scales();
       if constexpr (MT == 1) {
@@ -626,6 +707,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
         }
       }
     } else {
+      load_tile(t_begin, s_pl0, s_xr0, read_zones(t_begin));
       stage_scales();
       for (; t < t_end; t += 2) {
         step(t, s_pl0, s_xr0, s_pl1, s_xr1);
@@ -659,7 +741,8 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   // leave their sums in the staging area, free now, one slot per wave.
   auto owns = [&](int mt) { return kw == mt % KW; };  // wave-uniform
   if (KW > 1) {
-    auto red_slot = [&](int i) -> f32x4_t* {  // wave slots are spread over the plane slots
+    auto red_slot = [&](int i) -> f32x4_t* {  // wave slots are spread over the plane slots (direct: in the staged x)
+      if constexpr (DIRECT) return reinterpret_cast<f32x4_t*>(s_xs + i * RED_SLOT);
       unsigned char* base = i < RED_PER ? s_pl0 : (PF == 1 || i < 2 * RED_PER) ? s_pl1 : s_pl2;
       return reinterpret_cast<f32x4_t*>(base + (i % RED_PER) * RED_SLOT);
     };
@@ -713,7 +796,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
   // Apart from the stores of the sums, whose registers a branch around them
   // would spill.
   static_assert(KW > 1, "the reduction's barriers precede this read");
-  const bool late = s_late != 0;  // block-uniform
+  const bool late = !DIRECT && s_late != 0;  // block-uniform
   auto poison = [&]() {
     __builtin_amdgcn_s_waitcnt(0);  // the stores of the sums
 #pragma unroll 1
@@ -885,7 +968,6 @@ __global__ __launch_bounds__(256) void sigma_kernel(const uint16_t* __restrict__
 
 DecodePlan plan_decode(int64_t M, int64_t K, int64_t N, int max_bits, bool dense, bool wide) {
   DecodePlan pl{};
-  pl.wide = wide;
   pl.mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
   const int64_t NW = N / 16, T = K / 32;
   const int64_t bytes_per_split = M * N * (int64_t)sizeof(float);
@@ -919,7 +1001,7 @@ DecodePlan plan_decode(int64_t M, int64_t K, int64_t N, int max_bits, bool dense
   // line qkv 16.4 / 16.9, o_proj 14.1 / 15.5).  Graded batches read fewer
   // planes and are bound by their unpacking (gate_up 29.9 / 33.5 us).
   choose(1);
-  if (wide && dense && pl.mt <= 2) {
+  if (wide && dense && pl.mt <= 2 && !(pl.mt == 1 && max_bits == 2)) {
     choose(2);
     if (splits * 16 * pl.mt * 4 * 10 > 3 * K * max_bits / 8) choose(1);
   }
@@ -931,16 +1013,42 @@ DecodePlan plan_decode(int64_t M, int64_t K, int64_t N, int max_bits, bool dense
   pl.splits = (int)splits;
   pl.tiles_per_split = (int)tps;
   pl.workspace = splits > 1 ? (size_t)(splits * bytes_per_split) : 0;
+  // Up to 16 rows, waves that load their own words (twice the requests, but no
+  // handshake per tile and no LDS round trip) are faster than shared tiles
+  // where a tile or a wave's share of the K range is small, and, graded, where
+  // the shared tiles come by 4-byte loads.  16 rows, fp16, shared / direct us:
+  //   2 bits: down 14.3 / 13.4 dense, 15.2 / 14.0 graded; 4096 x 28688 24.1 /
+  //     22.5 and 25.9 / 24.3; but dense gate_up (2048 rows a block) 21.2 / 22.6
+  //   graded, rows not 16-byte aligned: 2080 x 6160 13.8 / 12.6, 4096 x 28688
+  //     36.1 / 33.6
+  //   graded, short K ranges: o_proj (256 rows a block) 12.1 / 11.7, qkv (416)
+  //     13.7 / 13.7, in 4 bits 12.7 / 12.4; longer ones down (896) 18.4 / 19.1,
+  //     gate_up (2048) 29.2 / 35.5
+  pl.load_words = wide ? 4 : 1;
+  const bool direct = dense ? max_bits == 2 && (!wide || tps <= 32) : max_bits == 2 || !wide || tps <= 16;
+  if (pl.mt == 1 && direct) pl.load_words = 0;
   return pl;
 }
 
 template <typename DT, int MT, int Z>
 static void launch_decode_t(const DecodeParams& p, const DecodePlan& pl, bool dense, hipStream_t st) {
   const dim3 grid(pl.col_blocks * pl.splits), block(64 * kDecodeWaves);
-  auto kernel = dense ? decode_kernel<DT, MT, Z, true, false, 1> : decode_kernel<DT, MT, Z, false, false, 1>;
-  if (pl.wide) kernel = dense ? decode_kernel<DT, MT, Z, true, true, 1> : decode_kernel<DT, MT, Z, false, true, 1>;
-  if constexpr (MT <= 2)
-    if (pl.cg == 2) kernel = decode_kernel<DT, MT, Z, true, true, 2>;  // (dense only: plan_decode)
+  // (which of the forms exist: plan_decode)
+  auto kernel = decode_kernel<DT, MT, Z, true, 4, 1>;
+  if constexpr (MT == 1) {
+    if (!dense) kernel = decode_kernel<DT, MT, Z, false, 0, 1>;
+    if constexpr (Z == 1) {
+      if (dense && pl.load_words == 0) kernel = decode_kernel<DT, MT, Z, true, 0, 1>;
+    } else {
+      if (!dense && pl.load_words == 4) kernel = decode_kernel<DT, MT, Z, false, 4, 1>;
+      if (dense && pl.load_words == 1) kernel = decode_kernel<DT, MT, Z, true, 1, 1>;
+    }
+  } else {
+    if (!dense) kernel = decode_kernel<DT, MT, Z, false, 4, 1>;
+    if (pl.load_words == 1) kernel = dense ? decode_kernel<DT, MT, Z, true, 1, 1> : decode_kernel<DT, MT, Z, false, 1, 1>;
+  }
+  if constexpr (MT <= 2 && (MT == 2 || Z > 1))
+    if (pl.cg == 2) kernel = decode_kernel<DT, MT, Z, true, 4, 2>;  // (dense only)
   launch_main_kernel(kernel, grid, block, st, p);
 }
 

@@ -46,7 +46,7 @@ constexpr int kTilePolls = 1 << 20;
 struct DecodePlan {
   int mt;      // 16-row m-tiles: 1, 2 or 4 (M <= 16, 32, 64)
   int cg;      // decode kernel: groups of 16 word columns per block
-  bool wide;   // decode kernel: 16-byte plane loads
+  int load_words;  // decode kernel: words per lane and plane load into LDS (4 or 1), or 0: into registers
   int splits;
   int tiles_per_split;
   int col_blocks;
