@@ -995,15 +995,19 @@ DecodePlan plan_decode(int64_t M, int64_t K, int64_t N, int max_bits, bool dense
   };
   // Dense batches of up to 32 rows are bound by the plane traffic, which
   // blocks of 32 word columns read in whole 128-byte lines, for twice the K
-  // ranges and so twice the partial sums: taken where those stay below 0.3 of
-  // the plane bytes (16 rows, 16 / 32 columns: gate_up 46 / 36 us, down 25.8 /
-  // 23.0, Llama-3-70B gate_up 147 / 126; 24 rows gate_up 49 / 42; above the
-  // line qkv 16.4 / 16.9, o_proj 14.1 / 15.5).  Graded batches read fewer
-  // planes and are bound by their unpacking (gate_up 29.9 / 33.5 us).
+  // ranges and so twice the partial sums.  6 and 8 bits: taken where those stay
+  // below 0.3 of the plane bytes (16 / 32 columns, us: 16 rows gate_up 46 / 36,
+  // down 25.8 / 23.0, Llama-3-70B gate_up 147 / 126, 24 rows gate_up 49 / 42;
+  // above the line qkv 16.4 / 16.9, o_proj 14.1 / 15.5).  4 bits: up to 16 rows
+  // and below 0.2 (gate_up 28.7 / 26.6; down, at 0.29, 17.0 / 18.1; 24 rows
+  // gate_up 30.2 / 35.1, Llama-3-70B down 55.4 / 65.8).  2 bits: never (gate_up
+  // 21.2 / 24.7).  Graded batches read fewer planes and are bound by their
+  // unpacking (gate_up 29.9 / 33.5).
   choose(1);
-  if (wide && dense && pl.mt <= 2 && !(pl.mt == 1 && max_bits == 2)) {
+  const int64_t percent = max_bits >= 6 ? 30 : (max_bits == 4 && pl.mt == 1) ? 20 : 0;
+  if (wide && dense && pl.mt <= 2 && percent > 0) {
     choose(2);
-    if (splits * 16 * pl.mt * 4 * 10 > 3 * K * max_bits / 8) choose(1);
+    if (splits * 16 * pl.mt * 4 * 100 > percent * K * max_bits / 8) choose(1);
   }
   if (splits < 1) splits = 1;
   int64_t tps = (T + splits - 1) / splits;
@@ -1047,7 +1051,7 @@ static void launch_decode_t(const DecodeParams& p, const DecodePlan& pl, bool de
     if (!dense) kernel = decode_kernel<DT, MT, Z, false, 4, 1>;
     if (pl.load_words == 1) kernel = dense ? decode_kernel<DT, MT, Z, true, 1, 1> : decode_kernel<DT, MT, Z, false, 1, 1>;
   }
-  if constexpr (MT <= 2 && (MT == 2 || Z > 1))
+  if constexpr (MT == 1 ? Z >= 2 : MT == 2 && Z >= 3)
     if (pl.cg == 2) kernel = decode_kernel<DT, MT, Z, true, 4, 2>;  // (dense only)
   launch_main_kernel(kernel, grid, block, st, p);
 }
