@@ -104,10 +104,14 @@ def test_product_graded_from_producer_statistic(M, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
-@pytest.mark.parametrize("M,K", [(2064, 4104), (1030, 8192), (17, 520)])
+@pytest.mark.parametrize("M,K", [(2064, 4104), (1030, 8192), (17, 520), (2064, 8200), (40, 8), (33, 504), (2064, 512),
+                                 (70, 1016), (2064, 1024), (33, 1032)])
 def test_large_batches(M, K, dtype):
-    """Batches whose blocks take several 512-column pieces (the norm) or four
-    rows per wave (the activation), ragged at the last piece and the last rows."""
+    """Batches whose blocks take several 512-column pieces (the norm: two at 2064 x
+    4104 and 1030 x 8192, four at 2064 x 8200, which use each buffer of maxima
+    twice) or four rows per wave (the activation), ragged at the last piece and
+    the last rows; rows around the widths of one and two runs of 512 columns,
+    which the norm keeps in flight differently."""
     from grinqh.producer import rmsnorm_sigma, silu_mul_sigma
     rng = np.random.default_rng(M * K)
     x, r, w = _rand(rng, (M, K), dtype, 3.0), _rand(rng, (M, K), dtype), _rand(rng, (K,), dtype)

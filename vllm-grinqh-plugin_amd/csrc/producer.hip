@@ -16,6 +16,8 @@
 // activation dtype and its fp32 square enters the variance; the normalised
 // value is rounded to the dtype before the weight multiply; silu is computed
 // in fp32 and rounded before the multiply by the up half.
+#include <type_traits>
+
 #include "grinqh_common.h"
 #include "grinqh_launch.h"
 
@@ -66,14 +68,19 @@ __device__ __forceinline__ void store_chunk_maxima(ProducerRows& s_abs, const fl
 // the column maxima.  32 rows x 4096 with the residual: 21.0 ->
 // 6.6 us (256 threads, 16 of them sharing a row and walking it with one load
 // in flight); 4096 rows x 8192: 138 -> 62 us (4.3 TB/s).
+// BATCH: runs of 512 columns in flight for the variance.  Rows of up to 1024
+// columns take 2, and of up to 512 the one run that the block's piece has loaded
+// already: with 8 they summed up to 7 runs of zeros, and the 64 registers of
+// those left one block per CU.  The loop is written once with and once without
+// the residual.  Without it, us: 16 rows x 256 5.6 -> 3.5, 8192 x 256 11.1 ->
+// 6.2, 4096 x 1024 12.6 -> 8.0, 16 x 4096 6.0 -> 5.0.
 // Since every column block reads whole rows of residual_in, the sum goes to a
 // separate residual_out (writing it back in place would race with those reads).
-template <typename DT>
+template <typename DT, int BATCH>
 __global__ __launch_bounds__(kProducerThreads) void rmsnorm_sigma_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ residual,
     uint16_t* __restrict__ residual_out, const uint16_t* __restrict__ weight, float eps, uint16_t* __restrict__ y,
     float* __restrict__ sigma_chunks, int M, int K, int pieces) {
-  constexpr int BATCH = 8;
   __shared__ ProducerRows s_abs[2];
   const int lane = threadIdx.x & 63;
   const int row = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -99,25 +106,38 @@ __global__ __launch_bounds__(kProducerThreads) void rmsnorm_sigma_kernel(
     float ss[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) ss[e] = 0.f;
-    for (int k0 = 8 * lane; k0 < K; k0 += 512 * BATCH) {
-      u32x4_t xa[BATCH], ra[BATCH];
+    auto add = [&](auto with_residual, const u32x4_t& xa, const u32x4_t& ra) {
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i) {
-        const bool in = k0 + 512 * i < K;
-        xa[i] = in ? *reinterpret_cast<const u32x4_t*>(xr + k0 + 512 * i) : zero;
-        ra[i] = in && rr != nullptr ? *reinterpret_cast<const u32x4_t*>(rr + k0 + 512 * i) : zero;
-      }
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i)
+        for (int h = 0; h < 2; ++h) {
+          float v = to_f32<DT>((uint16_t)(xa[q] >> (16 * h)));
+          if constexpr (decltype(with_residual)::value)
+            v = to_f32<DT>(from_f32<DT>(v + to_f32<DT>((uint16_t)(ra[q] >> (16 * h)))));
+          ss[2 * q + h] = fmaf(v, v, ss[2 * q + h]);
+        }
+    };
+    auto add_row = [&](auto with_residual) {
+      if constexpr (BATCH == 1) {
+        add(with_residual, a, r);
+      } else {
+        for (int k0 = 8 * lane; k0 < K; k0 += 512 * BATCH) {
+          u32x4_t xa[BATCH], ra[BATCH];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            float v = to_f32<DT>((uint16_t)(xa[i][q] >> (16 * h)));
-            if (rr != nullptr) v = to_f32<DT>(from_f32<DT>(v + to_f32<DT>((uint16_t)(ra[i][q] >> (16 * h)))));
-            ss[2 * q + h] = fmaf(v, v, ss[2 * q + h]);
+          for (int i = 0; i < BATCH; ++i) {
+            const bool in = k0 + 512 * i < K;
+            xa[i] = in ? *reinterpret_cast<const u32x4_t*>(xr + k0 + 512 * i) : zero;
+            ra[i] = decltype(with_residual)::value && in ? *reinterpret_cast<const u32x4_t*>(rr + k0 + 512 * i) : zero;
           }
-    }
+#pragma unroll
+          for (int i = 0; i < BATCH; ++i) add(with_residual, xa[i], ra[i]);
+        }
+      }
+    };
+    if (rr != nullptr)
+      add_row(std::true_type{});
+    else
+      add_row(std::false_type{});
 #pragma unroll
     for (int e = 4; e >= 1; e >>= 1)
 #pragma unroll
@@ -233,12 +253,14 @@ int launch_rmsnorm_sigma(const uint16_t* x, int64_t ldx, const uint16_t* residua
   const int pieces = producer_pieces(M, K);
   const dim3 grid((K + pieces * kProducerCols - 1) / (pieces * kProducerCols),
                   (M + kSigmaChunkRows - 1) / kSigmaChunkRows);
+  auto choose = [K](auto one, auto two, auto eight) {
+    return K <= kProducerCols ? one : (K <= 2 * kProducerCols ? two : eight);
+  };
+  auto kernel = choose(rmsnorm_sigma_kernel<F16, 1>, rmsnorm_sigma_kernel<F16, 2>, rmsnorm_sigma_kernel<F16, 8>);
   if (dtype == GRINQH_DTYPE_BF16)
-    hipLaunchKernelGGL(rmsnorm_sigma_kernel<BF16>, grid, dim3(kProducerThreads), 0, st, x, ldx, residual, residual_out, weight, eps, y,
-                       sigma_chunks, M, K, pieces);
-  else
-    hipLaunchKernelGGL(rmsnorm_sigma_kernel<F16>, grid, dim3(kProducerThreads), 0, st, x, ldx, residual, residual_out, weight, eps, y,
-                       sigma_chunks, M, K, pieces);
+    kernel = choose(rmsnorm_sigma_kernel<BF16, 1>, rmsnorm_sigma_kernel<BF16, 2>, rmsnorm_sigma_kernel<BF16, 8>);
+  hipLaunchKernelGGL(kernel, grid, dim3(kProducerThreads), 0, st, x, ldx, residual, residual_out, weight, eps, y,
+                     sigma_chunks, M, K, pieces);
   return hipGetLastError() == hipSuccess ? GRINQH_OK : GRINQH_ERR_HIP;
 }
 
