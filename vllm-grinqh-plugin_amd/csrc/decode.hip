@@ -16,17 +16,24 @@
 //             tiles
 //
 // What bounds it: at small shapes the launch, the prologue and the split-K
-// completion (about 10 us in all); in the loop, dense, the plane traffic, and
-// graded the unpacking VALU.  The plane words come through LDS by direct
-// buffer-to-LDS loads because of the traffic: with every wave loading its own
-// tiles into registers, the two waves that share a tile requested it twice, and
-// a stream of the same requests without arithmetic reached 2.1 TB/s (gate_up,
-// one MI355X); each tile requested once through 16-byte LDS loads reaches 3.4
-// TB/s with 16 word columns per block, 4.6 with 32, 5.4 with 64 (longer runs
-// of each plane line per block; a plain copy: 5.1).  The registers this frees
-// took bf16 above 16 rows from four waves per block to eight.  Measured,
-// product with its reduction: gate_up 16 rows dense 59.6 -> 36.2 us, 64 rows
-// 66.9 -> 58.8, in bf16 104.5 -> 56; Llama-3-70B gate_up 16 rows 178 -> 128.
+// completion (about 10 us in all); in the loop no single unit: the phases of a
+// tile (wait for its words, read them from LDS, unpack, multiply) follow one
+// another with two waves per SIMD.  Counters, gate_up: graded 47 rows 41 us,
+// VALU busy 39 % per SIMD, MFMA 14 %, waves waiting for memory or a dependency
+// 34 % and to issue 25 % of their time; dense 16 rows 28 us, 30 %, 5 %, 41 %,
+// 17 %, where the plane traffic (4.3 TB/s) is near what a copy reaches (5.1).
+//
+// The plane words come through LDS by direct buffer-to-LDS loads because of the
+// traffic: with every wave loading its own tiles into registers, the two waves
+// that share a tile requested it twice, and a stream of the same requests
+// without arithmetic reached 2.1 TB/s (gate_up, one MI355X); each tile requested
+// once through 16-byte LDS loads reaches 3.4 TB/s with 16 word columns per
+// block, 4.6 with 32, 5.4 with 64 (longer runs of each plane line per block).
+// The registers this frees took bf16 above 16 rows from four waves per block to
+// eight.  Measured, product with its reduction: gate_up 16 rows dense 59.6 ->
+// 36.2 us, 64 rows 66.9 -> 58.8, in bf16 104.5 -> 56; Llama-3-70B gate_up 16
+// rows 178 -> 128.  Up to 16 rows, where a tile or its K range is small, waves
+// load their own words all the same (plan_decode).
 //
 // Phase 1 (whole block): reduce the batch statistic of the block's rows from x
 // (unless given), grade every row (sigma = max_m |x|: zone bits, midpoint
@@ -37,7 +44,8 @@
 // the grading does not need has an offset past the buffer end, which leaves
 // zeros without a memory access.  A handshake through LDS flags per tile says
 // that all shares have arrived; then lane (c = lane & 15, q = lane >> 4) reads
-// the 8 x Z words of its 8 rows.  Code bytes are rebuilt branch-free:
+// the 8 x Z words of its 8 rows (or has loaded them itself, two tiles ahead).
+// Code bytes are rebuilt branch-free:
 // G_z = rot(D_z, 2z), H_j = field merge of the G_z, V_j = rot(H_j, -2j); then
 // turned into the MFMA B operand in one of two ways:
 //   - code bytes (5-16 rows, and bf16): fp16 B = u as the subnormal u*2^-24

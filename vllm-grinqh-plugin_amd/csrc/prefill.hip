@@ -49,7 +49,7 @@ __global__ __launch_bounds__(WAVES * 64, OCC) void prefill_kernel(PrefillParams 
   constexpr int AL = BM * CPR / NP;
   constexpr int RPT = BK / 16;      // rows per dequantizing thread
   constexpr int JPT = 4 * 256 / NP; // output dwords j per dequantizing thread
-  static_assert(!WS || (WAVES == 8 && PD % 2 == 0), "warp-specialised shape");
+  static_assert(!WS || (WAVES == 8 && PD == 2), "warp-specialised shape");
   static_assert(MTW >= 1 && AL >= 1 && RPT % 2 == 0 && JPT >= 1, "tile shape");
 
   __shared__ __align__(16) uint16_t s_a[2][BM * KP];
