@@ -269,6 +269,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, 1) void decode_kernel(DecodePara
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             xr, (__attribute__((address_space(3))) void*)(s_xs + t * 1024), 16, (int)off, 0, 0, 0);
       }
+      asm volatile("" ::: "memory");  // no load below moves above these: the wait for x counts on it
     }
     auto load_scales = [&]() {
 #pragma unroll
